@@ -123,10 +123,17 @@ TablesScope::~TablesScope() { g_override = prev; }
 // last column}, so each A entry costs one gather of a compact table (B.rows
 // x 16 B, cache-resident for the block-local column ranges of batched
 // inputs) instead of three dependent gathers into B's offsets and columns.
-// Rows of A up to kLongA entries take G lanes each; longer rows are listed
+// Rows of A up to long_a(G) entries take G lanes each; longer rows are listed
 // and taken by a whole workgroup each in a second pass, so one hub row does
 // not serialise its group for thousands of dependent loads.
-constexpr uint32_t kLongAIters = 32;  // iterations per lane before a row is "long"
+// Entries past which a row is "long": its own workgroup.  32 per lane, but
+// not below 256 (a listed row costs an atomic, and its group takes that many
+// entries in a few microseconds).
+constexpr uint32_t kMinLongA = 256;
+__host__ __device__ constexpr uint32_t long_a(int G) {
+  return 32u * (uint32_t)G > kMinLongA ? 32u * (uint32_t)G : kMinLongA;
+}
+static_assert(long_a(4) == kMinLongA, "the list is sized for the shortest long row");
 constexpr int kLongBlock = 256;
 
 __global__ __launch_bounds__(256) void k_brow_info(const uint32_t *__restrict__ b_rp,
@@ -151,54 +158,89 @@ struct AnaAcc {
   }
 };
 
+// G lanes per row, at most two 1024-thread workgroups per CU, grid-stride
+// over the rows with the next row's bounds loaded ahead.  The maxima cost
+// two same-address atomics per workgroup, about 12 ns each and one after
+// another over the whole chip, so the number of workgroups bounds the
+// kernel: with one 256-thread workgroup per 256 / G rows (up to 64 per CU)
+// it took 384 us on 262,144 rows of 8 entries and 290 us on 100,003 rows of
+// 24; now 47 and 36 us.
+constexpr int kAnaBlock = 1024;
+
 template <int G>
-__global__ __launch_bounds__(256) void k_analysis(
+__global__ __launch_bounds__(kAnaBlock) void k_analysis(
     const uint32_t *__restrict__ a_rp, const uint32_t *__restrict__ a_ci,
     uint32_t a_rows, const uint4 *__restrict__ info, uint32_t *__restrict__ products,
     uint32_t *__restrict__ max_b, uint32_t *__restrict__ avg_b,
     uint32_t *__restrict__ left, uint32_t *__restrict__ right,
     uint32_t *max_a_nnz, uint32_t *max_products, uint32_t *__restrict__ long_rows,
     uint32_t *long_count) {
-  constexpr int RPB = 256 / G;
+  constexpr int RPB = kAnaBlock / G;
   const int lig = threadIdx.x % G;
   uint32_t my_max_nnz = 0, my_max_prod = 0;
-  for (uint32_t r = blockIdx.x * RPB + threadIdx.x / G; r < a_rows;
-       r += gridDim.x * RPB) {
-    const uint32_t s = a_rp[r], e = a_rp[r + 1];
+  const uint64_t stride = (uint64_t)gridDim.x * RPB;
+  uint64_t r = (uint64_t)blockIdx.x * RPB + threadIdx.x / G;
+  uint32_t s = 0, e = 0;
+  if (r < a_rows) {
+    s = a_rp[r];
+    e = a_rp[r + 1];
+  }
+  while (r < a_rows) {
+    const uint64_t rn = r + stride;
+    uint32_t sn = 0, en = 0;
+    if (rn < a_rows) {
+      sn = a_rp[rn];
+      en = a_rp[rn + 1];
+    }
     const uint32_t n = e - s;
-    if (n > kLongAIters * G) {  // uniform over the group
+    if (n > long_a(G)) {  // uniform over the group
       if (lig == 0) {
-        long_rows[atomicAdd(long_count, 1u)] = r;
+        long_rows[atomicAdd(long_count, 1u)] = (uint32_t)r;
         my_max_nnz = max(my_max_nnz, n);
       }
-      continue;
+    } else {
+      AnaAcc acc;
+      uint32_t j = s + lig;
+      for (; j + 3 * G < e; j += 4 * G) {  // four independent gathers in flight
+        const uint32_t k0 = a_ci[j], k1 = a_ci[j + G], k2 = a_ci[j + 2 * G],
+                       k3 = a_ci[j + 3 * G];
+        const uint4 v0 = info[k0], v1 = info[k1], v2 = info[k2], v3 = info[k3];
+        acc.add(v0);
+        acc.add(v1);
+        acc.add(v2);
+        acc.add(v3);
+      }
+      // the rest (at most three), together: index 0 stands in for none
+      {
+        const bool h0 = j < e, h1 = j + G < e, h2 = j + 2 * G < e;
+        const uint32_t k0 = h0 ? a_ci[j] : 0u, k1 = h1 ? a_ci[j + G] : 0u,
+                       k2 = h2 ? a_ci[j + 2 * G] : 0u;
+        const uint4 none = make_uint4(0u, 0xFFFFFFFFu, 0u, 0u);
+        const uint4 v0 = h0 ? info[k0] : none, v1 = h1 ? info[k1] : none,
+                    v2 = h2 ? info[k2] : none;
+        acc.add(v0);
+        acc.add(v1);
+        acc.add(v2);
+      }
+      const uint32_t prod = group_sum(acc.prod, G);
+      const uint32_t mb = group_max(acc.mb, G);
+      const uint32_t lo = group_min(acc.lo, G);
+      const uint32_t hi = group_max(acc.hi, G);
+      if (lig == 0) {
+        products[r] = prod;
+        max_b[r] = mb;
+        avg_b[r] = n == 0 ? 0u : prod / n;
+        left[r] = lo;
+        right[r] = hi;
+        my_max_nnz = max(my_max_nnz, n);
+        my_max_prod = max(my_max_prod, prod);
+      }
     }
-    AnaAcc acc;
-    uint32_t j = s + lig;
-    for (; j + G < e; j += 2 * G) {  // two independent gathers in flight
-      const uint32_t k0 = a_ci[j], k1 = a_ci[j + G];
-      const uint4 v0 = info[k0], v1 = info[k1];
-      acc.add(v0);
-      acc.add(v1);
-    }
-    if (j < e) acc.add(info[a_ci[j]]);
-    const uint32_t prod = group_sum(acc.prod, G);
-    const uint32_t mb = group_max(acc.mb, G);
-    const uint32_t lo = group_min(acc.lo, G);
-    const uint32_t hi = group_max(acc.hi, G);
-    if (lig == 0) {
-      products[r] = prod;
-      max_b[r] = mb;
-      avg_b[r] = n == 0 ? 0u : prod / n;
-      left[r] = lo;
-      right[r] = hi;
-      my_max_nnz = max(my_max_nnz, n);
-      my_max_prod = max(my_max_prod, prod);
-    }
+    r = rn;
+    s = sn;
+    e = en;
   }
-  // one atomic per workgroup: same-address atomics serialise in L2, so
-  // one per wave over millions of rows would dominate the kernel
-  __shared__ uint32_t red[2][256 / kWave];
+  __shared__ uint32_t red[2][kAnaBlock / kWave];
   my_max_nnz = group_max(my_max_nnz, kWave);
   my_max_prod = group_max(my_max_prod, kWave);
   if (lane_id() == 0) {
@@ -207,7 +249,7 @@ __global__ __launch_bounds__(256) void k_analysis(
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 256 / kWave; ++w) {
+    for (int w = 1; w < kAnaBlock / kWave; ++w) {
       my_max_nnz = max(my_max_nnz, red[0][w]);
       my_max_prod = max(my_max_prod, red[1][w]);
     }
@@ -227,6 +269,7 @@ __global__ __launch_bounds__(kLongBlock) void k_analysis_long(
   __shared__ uint4 part[NW];
   const uint32_t nlong = *long_count;
   const int wid = threadIdx.x / kWave;
+  uint32_t my_max = 0;  // thread 0: one atomic per workgroup, not per row
   for (uint32_t i = blockIdx.x; i < nlong; i += gridDim.x) {
     const uint32_t r = long_rows[i];
     const uint32_t s = a_rp[r], e = a_rp[r + 1];
@@ -261,10 +304,11 @@ __global__ __launch_bounds__(kLongBlock) void k_analysis_long(
       avg_b[r] = t.x / (e - s);
       left[r] = t.z;
       right[r] = t.w;
-      if (max_products) atomicMax(max_products, t.x);
+      my_max = max(my_max, t.x);
     }
     __syncthreads();  // part[] is reused by the next row
   }
+  if (threadIdx.x == 0 && my_max && max_products) atomicMax(max_products, my_max);
 }
 
 __global__ void k_zero3(uint32_t *a, uint32_t *b, uint32_t *c) {
@@ -311,7 +355,7 @@ int launch_fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t s) {
 }
 
 size_t analysis_temp_bytes(uint64_t a_rows, uint64_t a_nnz, uint64_t b_rows) {
-  const uint64_t nlong = std::min<uint64_t>(a_rows, a_nnz / (kLongAIters * 4) + 1);
+  const uint64_t nlong = std::min<uint64_t>(a_rows, a_nnz / 128 + 1);
   return (b_rows + 1) * 16 + 256 + nlong * 4;
 }
 
@@ -343,22 +387,23 @@ int launch_analysis(const DevCsr &A, const DevCsr &B, const RowInfo &ri,
                        dim3(256), 0, s, B.rp, B.ci, (uint32_t)B.rows, info);
   const double avg = (double)A.nnz / (double)A.rows;
   const uint32_t rows = (uint32_t)A.rows;
-  // grid-stride over at most 64 workgroups per CU
-  const uint32_t max_grid = 64 * std::max<uint32_t>(tables().num_cu, 1);
-#define GO(G)                                                                 \
-  hipLaunchKernelGGL(k_analysis<G>,                                           \
-                     dim3(std::min<uint32_t>(cdiv(rows, 256 / G), max_grid)), \
-                     dim3(256), 0, s, A.rp, A.ci, rows, info,                 \
-                     ri.products, ri.max_b, ri.avg_b, ri.left, ri.right,      \
+  // at most the resident workgroups (two per CU); lanes for about half of the
+  // average row, whose entries each lane then loads together
+  const uint32_t max_grid = 2 * std::max<uint32_t>(tables().num_cu, 1);
+#define GO(G)                                                                       \
+  hipLaunchKernelGGL(k_analysis<G>,                                                 \
+                     dim3(std::min<uint32_t>(cdiv(rows, kAnaBlock / G), max_grid)), \
+                     dim3(kAnaBlock), 0, s, A.rp, A.ci, rows, info,                 \
+                     ri.products, ri.max_b, ri.avg_b, ri.left, ri.right,            \
                      max_a_nnz, max_products, long_rows, long_count)
-  if (avg <= 4) GO(4);
-  else if (avg <= 8) GO(8);
-  else if (avg <= 16) GO(16);
-  else if (avg <= 32) GO(32);
+  if (avg <= 8) GO(4);
+  else if (avg <= 16) GO(8);
+  else if (avg <= 32) GO(16);
+  else if (avg <= 64) GO(32);
   else GO(64);
 #undef GO
-  // a row is long only past kLongAIters * 4 entries, so the list holds at
-  // most nnz / (kLongAIters * 4) rows, the size analysis_temp_bytes gives it
+  // a row is long only past kMinLongA entries, so the list holds at most
+  // nnz / kMinLongA rows; analysis_temp_bytes gives it twice that
   hipLaunchKernelGGL(k_analysis_long, dim3(1024), dim3(kLongBlock), 0, s, A.rp, A.ci, info,
                      ri.products, ri.max_b, ri.avg_b, ri.left, ri.right, max_products,
                      long_rows, long_count);
