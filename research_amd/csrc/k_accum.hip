@@ -666,7 +666,7 @@ __host__ __device__ inline HashLayout hash_layout(uint32_t S, uint32_t nwaves) {
   p += 4 * L.nmax;
   L.off_ci = p;
   p += 2 * L.nmax;
-  p = (p + 3) & ~3u;
+  p = (p + 7) & ~7u;  // read as bucket counters, eight bytes at a time
   L.off_cnt = p;
   p += nwaves * 512;
   L.bytes = p;
@@ -811,6 +811,71 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
     }
     if (o.nnz && threadIdx.x == 0) o.nnz[r] = n;
     return;
+  }
+  // Wider rows are ordered by column bucket: the top bits of the span give
+  // each key one of 256 buckets per wave, a count, a scan and a scatter group
+  // the keys by bucket, and a key's place is its bucket's start plus the
+  // smaller keys beside it in the bucket (about one for spread columns).  The
+  // radix sort below takes three passes with eight ballots per 64 keys each:
+  // it made the kernel bound by its vector instructions (7384 per row of 576
+  // products, 78% of the issue slots; with buckets 2260).  It stays for rows
+  // whose columns crowd into few buckets, where comparing within one costs
+  // more.  (85,720 Erdos-Renyi rows of 576 products, 256 threads: 1393 -> 730
+  // us; R-MAT 2^18's rows of the largest tables, 1024 threads: 2553 -> 1429.)
+  if (!hdr[1]) {
+    constexpr uint32_t kCrowded = 192;  // keys of one bucket
+    uint32_t *bw = reinterpret_cast<uint32_t *>(smem + L.off_cnt);  // two buckets a word
+    const uint16_t *bend = reinterpret_cast<const uint16_t *>(bw);
+    uint2 *mine4 = reinterpret_cast<uint2 *>(bw) + threadIdx.x;  // a thread's four buckets
+    *mine4 = make_uint2(0u, 0u);
+    if (threadIdx.x == 0) hdr[4] = 0;
+    // BS / 64 * 256 buckets = 4 BS
+    constexpr int kLogBuckets = __builtin_ctz(BS) + 2;
+    const int span_bits = rh.right > lo ? 32 - __clz(rh.right - lo) : 0;
+    const uint32_t sh = (uint32_t)max(0, span_bits - kLogBuckets);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < S; i += BS) {
+      const uint32_t kk = keys[i];
+      if (kk != kEmpty) {
+        const uint32_t b = (kk - lo) >> sh;
+        atomicAdd(&bw[b >> 1], 1u << (16 * (b & 1)));
+      }
+    }
+    __syncthreads();
+    const uint2 cw = *mine4;
+    const uint32_t n0 = cw.x & 0xFFFFu, n1 = cw.x >> 16, n2 = cw.y & 0xFFFFu, n3 = cw.y >> 16;
+    if (max(max(n0, n1), max(n2, n3)) > kCrowded) hdr[4] = 1;
+    uint32_t n;
+    const uint32_t st = block_excl_sum(n0 + n1 + n2 + n3, dsum, &n);
+    *mine4 = make_uint2(st | (st + n0) << 16, (st + n0 + n1) | (st + n0 + n1 + n2) << 16);
+    if (n > L.nmax || (EST && n > cap)) {
+      if (threadIdx.x == 0) o.ovf_rows[atomicAdd(o.ovf_count, 1u)] = r;
+      return;
+    }
+    __syncthreads();
+    if (!hdr[4]) {
+      // each bucket's start moves to its end as its keys are placed
+      for (uint32_t i = threadIdx.x; i < S; i += BS) {
+        const uint32_t kk = keys[i];
+        if (kk != kEmpty) {
+          const uint32_t b = (kk - lo) >> sh, half = 16 * (b & 1);
+          const uint32_t pos = (atomicAdd(&bw[b >> 1], 1u << half) >> half) & 0xFFFFu;
+          ck[pos] = kk;
+          ci[pos] = (uint16_t)i;
+        }
+      }
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < n; i += BS) {
+        const uint32_t kk = ck[i], b = (kk - lo) >> sh;
+        const uint32_t s0 = b ? bend[b - 1] : 0u, s1 = bend[b];
+        uint32_t pos = s0;
+        for (uint32_t t = s0; t < s1; ++t) pos += ck[t] < kk ? 1u : 0u;
+        o.cols[off + pos] = kk;
+        o.vals[off + pos] = (T)vals[ci[i]];
+      }
+      if (o.nnz && threadIdx.x == 0) o.nnz[r] = n;
+      return;
+    }
   }
   // compaction of occupied slots; keys relative to the row's first column,
   // so the sort needs only the bits of the row's column span
