@@ -72,6 +72,9 @@ int launch_fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t s);
 // bounds = {0, *count}: the row range of a device-counted list
 int launch_count_bounds(const uint32_t *count, uint32_t *bounds, hipStream_t s);
 size_t scan_temp_bytes(uint64_t n);
+// what a scan of n entries cannot do without (the documented limit of
+// oc_analysis_noalloc counts this)
+size_t scan_temp_bytes_min(uint64_t n);
 int launch_scan_u32(const uint32_t *in, uint64_t *out, uint64_t n, void *temp,
                     hipStream_t s);
 int launch_murmur(const uint32_t *cols, uint32_t *out, uint64_t n,

@@ -27,10 +27,13 @@ namespace oc {
   } while (0)
 
 constexpr size_t kNoAllocScratchBytes = 32u << 20;
+// room beyond the limit for the part of the scan's partials that the limit
+// does not count (scan_temp_bytes against scan_temp_bytes_min)
+constexpr size_t kScanSlackBytes = 8192;
 
 // Host code never uses this name as an address: the device address of each
 // device's copy comes from hipGetSymbolAddress (scratch_ptr below).
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes + kScanSlackBytes];
 
 namespace {
 
@@ -90,11 +93,13 @@ extern "C" int oc_analysis_noalloc(const oc_csr *dA, const oc_csr *dB, uint32_t 
   // layout: 256 B of counters, the scan partials, the analysis temporaries
   const size_t scan_b = (scan_temp_bytes(dA->rows + 1) + 255) & ~(size_t)255;
   const size_t ana_b = analysis_temp_bytes(dA->rows, dA->nnz, dB->rows);
-  const size_t need = 256 + scan_b + ana_b;
+  const size_t need = 256 + ((scan_temp_bytes_min(dA->rows + 1) + 255) & ~(size_t)255) + ana_b;
   OC_REQUIRE(need <= kNoAllocScratchBytes,
              "oc_analysis_noalloc: these operands need %zu bytes of scratch, beyond the "
              "%zu-byte limit (use oc_analysis)",
              need, kNoAllocScratchBytes);
+  OC_REQUIRE(256 + scan_b + ana_b <= kNoAllocScratchBytes + kScanSlackBytes,
+             "internal: the scan's partials outgrew the scratch array's slack");
   void *base = nullptr;
   OC_TRY(scratch_ptr(&base));
   uint8_t *p = (uint8_t *)base;
