@@ -369,7 +369,7 @@ __device__ __forceinline__ uint32_t list_heavy(const KA &a, const RowHead &rh, u
 }
 
 // Persistent row loop over the rows [bounds[0], bounds[1]) of a bin list:
-// chunks of kClaimRows rows claimed from *claim (zeroed before the launch).
+// chunks of kClaimRows rows claimed from *claim (zeroed before the launches).
 // A workgroup that starts late or draws costly rows takes fewer chunks;
 // each workgroup striding over a fixed share of the rows ran the bins
 // 10-40% slower than launching one workgroup per row.  One loop latch,
@@ -403,6 +403,25 @@ __device__ __forceinline__ void claim_rows(const uint32_t *__restrict__ bounds, 
     const uint32_t e = min(b1, b0 + c + chunk);
     for (uint32_t i = b0 + c; i < e; ++i) {
       row(i);
+      __syncthreads();  // the next row re-initialises the LDS
+    }
+  }
+}
+
+// The rows of a bin kernel: the workgroup's own (one workgroup per row), the
+// rows [bounds[0], bounds[1]) by claims, or, without a claim counter, by a
+// stride of the grid (which is then about as many workgroups as rows).
+template <typename F>
+__device__ __forceinline__ void bin_rows(const uint32_t *__restrict__ bounds, uint32_t *claim,
+                                         F &&row) {
+  if (!bounds) {
+    row(blockIdx.x);
+  } else if (claim) {
+    claim_rows(bounds, claim, row);
+  } else {
+    const uint32_t b0 = bounds[0], b1 = bounds[1];
+    for (uint64_t i = (uint64_t)b0 + blockIdx.x; i < b1; i += gridDim.x) {
+      row((uint32_t)i);
       __syncthreads();  // the next row re-initialises the LDS
     }
   }
@@ -545,11 +564,7 @@ template <int BS>
 __global__ __launch_bounds__(BS) void k_sym_hash(KArgs<float> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, uint32_t S, uint32_t limit, uint32_t *__restrict__ nnz, uint32_t *ovf_rows, uint32_t *ovf_count,
     uint32_t *claim) {
-  if (!bounds) {
-    sym_hash_row<BS>(a, rows[blockIdx.x], S, limit, nnz, ovf_rows, ovf_count);
-    return;
-  }
-  claim_rows(bounds, claim, [&](uint32_t i) {
+  bin_rows(bounds, claim, [&](uint32_t i) {
     sym_hash_row<BS>(a, rows[i], S, limit, nnz, ovf_rows, ovf_count);
   });
 }
@@ -632,11 +647,7 @@ template <int BS, bool WIN = false>
 __global__ __launch_bounds__(BS) void k_sym_dense(KArgs<float> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, uint32_t *__restrict__ nnz, const uint64_t *__restrict__ bmoff, uint4 *__restrict__ bm,
     uint32_t wbits, uint32_t *claim) {
-  if (!bounds) {
-    sym_dense_row<BS, WIN>(a, rows[blockIdx.x], nnz, bmoff, bm, wbits);
-    return;
-  }
-  claim_rows(bounds, claim, [&](uint32_t i) {
+  bin_rows(bounds, claim, [&](uint32_t i) {
     sym_dense_row<BS, WIN>(a, rows[i], nnz, bmoff, bm, wbits);
   });
 }
@@ -918,11 +929,7 @@ __global__ __launch_bounds__(BS) void k_num_hash(KArgs<T> a, const uint32_t *__r
     const uint32_t *__restrict__ bounds, const uint32_t *__restrict__ err, HashLayout L, KOut<T> o, int key_bits,
     uint32_t *claim) {
   if (err && *err) return;  // the capacity check failed: write nothing
-  if (!bounds) {
-    num_hash_row<BS, T, EST>(a, rows[blockIdx.x], L, o, key_bits);
-    return;
-  }
-  claim_rows(bounds, claim, [&](uint32_t i) {
+  bin_rows(bounds, claim, [&](uint32_t i) {
     num_hash_row<BS, T, EST>(a, rows[i], L, o, key_bits);
   });
 }
@@ -1042,11 +1049,7 @@ __global__ __launch_bounds__(BS) void k_num_dense(KArgs<T> a, const uint32_t *__
     const uint32_t *__restrict__ bounds, const uint32_t *__restrict__ err, KOut<T> o,
     uint32_t *claim) {
   if (err && *err) return;  // the capacity check failed: write nothing
-  if (!bounds) {
-    num_dense_row<BS, T, EST>(a, rows[blockIdx.x], o);
-    return;
-  }
-  claim_rows(bounds, claim, [&](uint32_t i) { num_dense_row<BS, T, EST>(a, rows[i], o); });
+  bin_rows(bounds, claim, [&](uint32_t i) { num_dense_row<BS, T, EST>(a, rows[i], o); });
 }
 
 // ============================================================== windowed
@@ -1962,25 +1965,36 @@ static uint32_t persistent_grid(K kernel, uint32_t bs, size_t lds) {
   return std::max<uint32_t>(1, t.num_cu) * (uint32_t)per_cu;
 }
 
-// The grid of a persistent launch over a bin: every resident workgroup, or
-// at most one per row when the host knows the bin's size (nrows > 0).
+// How a bin's rows reach its workgroups.
+//  - One workgroup per row when the host knows the bin (sel.first, nrows)
+//    and more than two workgroups fit a CU: the hardware then hides the gap
+//    between one row's workgroup and the next, and claims cost more than
+//    they gain (R-MAT 2^20: k_num_dense 0.11 -> 0.46 ms with claims).
+//  - With one or two per CU the CU idles in that gap, and claims win
+//    (k_sym_dense<1024> 32.6 -> 26.1 ms): every resident workgroup, or at
+//    most one per row.
+//  - A whole-path replay knows only the planned size.  With more than two
+//    workgroups per CU it runs that many (at least the resident ones), which
+//    stride over the bin's present rows.  Claims there are bound by the
+//    counter, about 12 ns each one after another: 274,832 rows of the
+//    smallest numeric table took 1518 us against 533 us with a workgroup per
+//    row, now 314 us.
+struct BinGrid {
+  uint32_t grid;
+  const uint32_t *rows, *bounds;
+  uint32_t *claim;
+};
 template <typename K>
-static uint32_t claim_grid(K kernel, uint32_t bs, size_t lds, uint32_t nrows) {
+static BinGrid bin_grid(const RowSel &sel, const uint32_t *rows, uint32_t nrows, K kernel,
+                        uint32_t bs, size_t lds) {
+  if (!sel.bounds) return BinGrid{nrows, rows, nullptr, nullptr};
   const uint32_t full = persistent_grid(kernel, bs, lds);
-  return nrows ? std::min<uint32_t>(full, nrows) : full;
-}
-
-// A bin launch whose host knows the bin (sel.first, nrows) runs one
-// workgroup per row when more than two workgroups fit a CU: the hardware
-// then hides the gap between one row's workgroup and the next, and the
-// claims cost more than they gain (R-MAT 2^20: k_num_dense 0.11 -> 0.46 ms
-// persistent).  With one or two per CU the CU idles in that gap, and the
-// claims win (k_sym_dense<1024> 32.6 -> 26.1 ms).
-template <typename K>
-static bool run_persistent(const RowSel &sel, uint32_t nrows, K kernel, uint32_t bs, size_t lds) {
-  if (!sel.bounds) return false;
-  if (!nrows || sel.first == ~0u) return true;
-  return persistent_grid(kernel, bs, lds) <= 2 * std::max<uint32_t>(1, tables().num_cu);
+  const bool many = full > 2 * std::max<uint32_t>(1, tables().num_cu);
+  if (many && nrows && sel.first != ~0u)
+    return BinGrid{nrows, rows + sel.first, nullptr, nullptr};
+  if (many && sel.planned)
+    return BinGrid{std::max(full, sel.planned), rows, sel.bounds, nullptr};
+  return BinGrid{nrows ? std::min(full, nrows) : full, rows, sel.bounds, sel.claim};
 }
 
 int launch_sym_hash(int bin, const AccArgs &a, const uint32_t *rows,
@@ -1994,13 +2008,10 @@ int launch_sym_hash(int bin, const AccArgs &a, const uint32_t *rows,
 #define GO(BS)                                                                \
   do {                                                                        \
     OC_TRY(set_lds(k_sym_hash<BS>, lds));                                     \
-    const bool per = run_persistent(sel, nrows, k_sym_hash<BS>, BS, lds);    \
-    const uint32_t grid = per ? claim_grid(k_sym_hash<BS>, BS, lds, nrows) : nrows; \
-    if (per) OC_TRY(zero_u32(sel.claim, 1, s));                               \
-    hipLaunchKernelGGL(k_sym_hash<BS>, dim3(grid), dim3(BS), lds, s, k,        \
-                       per || !sel.bounds ? rows : rows + sel.first,          \
-                       per ? sel.bounds : nullptr, S, std::min(limit, S), nnz, \
-                       ovf_rows, ovf_count, sel.claim);                       \
+    const BinGrid bg = bin_grid(sel, rows, nrows, k_sym_hash<BS>, BS, lds); \
+    hipLaunchKernelGGL(k_sym_hash<BS>, dim3(bg.grid), dim3(BS), lds, s, k,     \
+                       bg.rows, bg.bounds, S, std::min(limit, S), nnz,         \
+                       ovf_rows, ovf_count, bg.claim);                       \
   } while (0)
   BIN_DISPATCH(bin, GO)
 #undef GO
@@ -2019,13 +2030,10 @@ int launch_sym_dense(int dense_bin, const AccArgs &a, const uint32_t *rows,
 #define GO(BS)                                                                 \
   do {                                                                         \
     OC_TRY(set_lds(k_sym_dense<BS>, lds));                                     \
-    const bool per = run_persistent(sel, nrows, k_sym_dense<BS>, BS, lds);     \
-    const uint32_t grid = per ? claim_grid(k_sym_dense<BS>, BS, lds, nrows) : nrows; \
-    if (per) OC_TRY(zero_u32(sel.claim, 1, s));                                \
-    hipLaunchKernelGGL(k_sym_dense<BS>, dim3(grid), dim3(BS), lds, s, k,        \
-                       per || !sel.bounds ? rows : rows + sel.first,           \
-                       per ? sel.bounds : nullptr, nnz, bmoff, (uint4 *)bm, 0u, \
-                       sel.claim);                                             \
+    const BinGrid bg = bin_grid(sel, rows, nrows, k_sym_dense<BS>, BS, lds); \
+    hipLaunchKernelGGL(k_sym_dense<BS>, dim3(bg.grid), dim3(BS), lds, s, k,     \
+                       bg.rows, bg.bounds, nnz, bmoff, (uint4 *)bm, 0u,         \
+                       bg.claim);                                             \
   } while (0)
   BIN_DISPATCH(dense_bin, GO)
 #undef GO
@@ -2051,12 +2059,10 @@ int launch_sym_window(const AccArgs &a, const uint32_t *rows, uint32_t nrows,
   }
   const uint32_t wbits = (uint32_t)(((lds - 256) / 16 - 1) * 128);
   OC_TRY(set_lds(k_sym_dense<1024, true>, lds));
-  const bool per = run_persistent(sel, nrows, k_sym_dense<1024, true>, 1024, lds);
-  const uint32_t grid = per ? claim_grid(k_sym_dense<1024, true>, 1024, lds, nrows) : nrows;
-  if (per) OC_TRY(zero_u32(sel.claim, 1, s));
-  hipLaunchKernelGGL((k_sym_dense<1024, true>), dim3(grid), dim3(1024), lds, s,
-                     kargs<float>(a), per || !sel.bounds ? rows : rows + sel.first,
-                     per ? sel.bounds : nullptr, nnz, bmoff, (uint4 *)bm, wbits, sel.claim);
+  const BinGrid bg = bin_grid(sel, rows, nrows, k_sym_dense<1024, true>, 1024, lds);
+  hipLaunchKernelGGL((k_sym_dense<1024, true>), dim3(bg.grid), dim3(1024), lds, s,
+                     kargs<float>(a), bg.rows, bg.bounds, nnz, bmoff, (uint4 *)bm, wbits,
+                     bg.claim);
   LAUNCH_CHECK();
   return OC_OK;
 }
@@ -2075,13 +2081,10 @@ int launch_num_hash(int bin, const AccArgs &a, const uint32_t *rows,
 #define GO3(BS, T, E)                                                          \
   do {                                                                         \
     OC_TRY(set_lds(k_num_hash<BS, T, E>, L.bytes));                            \
-    const bool per = run_persistent(sel, nrows, k_num_hash<BS, T, E>, BS, L.bytes); \
-    const uint32_t grid = per ? claim_grid(k_num_hash<BS, T, E>, BS, L.bytes, nrows) : nrows; \
-    if (per) OC_TRY(zero_u32(sel.claim, 1, s));                                \
-    hipLaunchKernelGGL((k_num_hash<BS, T, E>), dim3(grid), dim3(BS), L.bytes,  \
-                       s, kargs<T>(a), per || !sel.bounds ? rows : rows + sel.first, \
-                       per ? sel.bounds : nullptr, sel.err, L, kout<T>(o), kb, \
-                       sel.claim);                                             \
+    const BinGrid bg = bin_grid(sel, rows, nrows, k_num_hash<BS, T, E>, BS, L.bytes); \
+    hipLaunchKernelGGL((k_num_hash<BS, T, E>), dim3(bg.grid), dim3(BS), L.bytes, \
+                       s, kargs<T>(a), bg.rows, bg.bounds, sel.err, L, kout<T>(o), kb, \
+                       bg.claim);                                             \
   } while (0)
 #define GO(BS)                                            \
   do {                                                    \
@@ -2115,12 +2118,9 @@ int launch_num_dense(int dense_bin, const AccArgs &a, const uint32_t *rows,
 #define GO3(BS, T, E)                                                           \
   do {                                                                          \
     OC_TRY(set_lds(k_num_dense<BS, T, E>, lds));                                \
-    const bool per = run_persistent(sel, nrows, k_num_dense<BS, T, E>, BS, lds); \
-    const uint32_t grid = per ? claim_grid(k_num_dense<BS, T, E>, BS, lds, nrows) : nrows; \
-    if (per) OC_TRY(zero_u32(sel.claim, 1, s));                                 \
-    hipLaunchKernelGGL((k_num_dense<BS, T, E>), dim3(grid), dim3(BS), lds, s,   \
-                       kargs<T>(a), per || !sel.bounds ? rows : rows + sel.first, \
-                       per ? sel.bounds : nullptr, sel.err, kout<T>(o), sel.claim); \
+    const BinGrid bg = bin_grid(sel, rows, nrows, k_num_dense<BS, T, E>, BS, lds); \
+    hipLaunchKernelGGL((k_num_dense<BS, T, E>), dim3(bg.grid), dim3(BS), lds, s, \
+                       kargs<T>(a), bg.rows, bg.bounds, sel.err, kout<T>(o), bg.claim); \
   } while (0)
 #define GO(BS)                                            \
   do {                                                    \

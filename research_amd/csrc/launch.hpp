@@ -162,11 +162,15 @@ struct NumOut {
 struct RowSel {
   const uint32_t *bounds = nullptr;
   const uint32_t *err = nullptr;
-  uint32_t *claim = nullptr;  // row-claim counter of the hash/dense bins (zeroed per launch)
+  uint32_t *claim = nullptr;  // this launch's row-claim counter (hash/dense bins), zeroed before it
   // the bin's first list entry when the host knows it (eager runs, which
   // pass the bin's row count): bins with many workgroups per CU then run
   // one workgroup per row from rows + first
   uint32_t first = ~0u;
+  // whole-path replays: the rows the bin held when it was planned.  Bins
+  // with many workgroups per CU then run about that many workgroups, each
+  // striding over the bin's present rows, and claim nothing.
+  uint32_t planned = 0;
 };
 
 // Symbolic: rows of one bin.  Overflowing rows (estimated-compaction hash

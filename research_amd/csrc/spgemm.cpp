@@ -256,7 +256,8 @@ struct oc_spgemm {
     DevCsr A{}, B{};
     RowInfo ri{};
     const uint32_t *brows = nullptr;
-    uint32_t hoff[kBinSlots + 1] = {0};
+    uint32_t hoff[kBinSlots + 1] = {0};   // numeric bins
+    uint32_t hoff1[kBinSlots + 1] = {0};  // symbolic bins
     NumOut o{};
     uint32_t *tile_ts = nullptr, *tile_tsw = nullptr;
     const uint32_t *block_base = nullptr;
@@ -461,11 +462,15 @@ struct Run {
     return a;
   }
 
-  // the row-claim counter of persistent bin launches (zeroed per launch)
+  // the row-claim counters of the persistent bin launches, one each
+  // (symbolic bin b: b, the recount of overflow rows: 14, numeric bin b:
+  // 16 + b), all cleared by one launch before the first of them
+  static constexpr uint32_t kClaims = 30, kClaimRecount = 14, kClaimNumeric = 16;
   uint32_t *claim_ctr = nullptr;
   int claims() {
-    if (!claim_ctr) OC_TRY(ar.get(&claim_ctr, 64));
-    return OC_OK;
+    if (claim_ctr) return OC_OK;
+    OC_TRY(ar.get(&claim_ctr, 64));
+    return launch_fill_u32(claim_ctr, kClaims, 0u, s);
   }
 
   int window_scratch() {
@@ -702,7 +707,8 @@ struct Run {
         return OC_ERR_INVALID;
       }
       if (boff)
-        OC_TRY(launch_num_hash(b, a, brows, n, o, s, RowSel{boff + b, nullptr, claim_ctr, hoff[b]}));
+        OC_TRY(launch_num_hash(b, a, brows, n, o, s,
+                               RowSel{boff + b, nullptr, claim_ctr + kClaimNumeric + b, hoff[b]}));
       else
         OC_TRY(launch_num_hash(b, a, brows + hoff[b], n, o, s));
     }
@@ -713,7 +719,7 @@ struct Run {
       if (!n) continue;
       if (boff)
         OC_TRY(launch_num_dense(b - 7, a, brows, n, o, s,
-                                RowSel{boff + b, nullptr, claim_ctr, hoff[b]}));
+                                RowSel{boff + b, nullptr, claim_ctr + kClaimNumeric + b, hoff[b]}));
       else
         OC_TRY(launch_num_dense(b - 7, a, brows + hoff[b], n, o, s));
     }
@@ -1116,14 +1122,14 @@ int Run::run_precise() {
     const uint32_t S = t.hash_sym[b];
     const uint32_t limit = d.use_est_symbolic ? S - S / 8 : S;
     OC_TRY(launch_sym_hash(b, a, brows, n, limit, nnz, ovf_rows, ovf, s,
-                           RowSel{boff + b, nullptr, claim_ctr, hoff[b]}));
+                           RowSel{boff + b, nullptr, claim_ctr + b, hoff[b]}));
   }
   fam("sym_hash", "symbolic_hash", false, brows + hoff[0], hoff[6] - hoff[0]);
   mk.mark("symbolic_hash");
   if (hoff[7] > hoff[6]) {
     OC_TRY(window_scratch());
     OC_TRY(launch_sym_window(a, brows, hoff[7] - hoff[6], h->max_a_nnz, nnz, win_scratch, s,
-                             RowSel{boff + 6, nullptr, claim_ctr, hoff[6]}, row_bmoff, row_bm));
+                             RowSel{boff + 6, nullptr, claim_ctr + 6, hoff[6]}, row_bmoff, row_bm));
   }
   fam("sym_window", "symbolic_window", false, brows + hoff[6], hoff[7] - hoff[6]);
   mk.mark("symbolic_window");
@@ -1135,7 +1141,7 @@ int Run::run_precise() {
       return OC_ERR_INVALID;
     }
     OC_TRY(launch_sym_dense(b - 7, a, brows, n, nnz, s, row_bmoff, row_bm,
-                            RowSel{boff + b, nullptr, claim_ctr, hoff[b]}));
+                            RowSel{boff + b, nullptr, claim_ctr + b, hoff[b]}));
   }
   fam("sym_dense", "symbolic_dense", false, brows + hoff[7], hoff[14] - hoff[7]);
   mk.mark("symbolic_dense");
@@ -1198,6 +1204,7 @@ int Run::run_precise() {
     p.ri = ri;
     p.brows = brows2;
     std::memcpy(p.hoff, hoff, sizeof(hoff));
+    std::memcpy(p.hoff1, h->bin1, sizeof(p.hoff1));
     p.o = o;
     p.tile_ts = tile_ts;
     p.tile_tsw = tile_tsw;
@@ -1871,7 +1878,8 @@ int replay_impl(oc_spgemm *h, hipStream_t s) {
   r.band.pref = p.band_pref;
   const uint32_t keep_max = h->max_a_nnz;
   h->max_a_nnz = p.max_a_nnz;
-  r.claim_ctr = p.err + 32;  // the plan's claim counter (no allocation here)
+  r.claim_ctr = p.err + 32;  // the plan's claim counters (no allocation here)
+  OC_TRY(launch_fill_u32(r.claim_ctr, Run::kClaims, 0u, s));
   int rc = r.numeric_bins(p.brows, p.hoff, p.o, true, p.boff2);
   if (rc == OC_OK) rc = r.band_numeric(p.o);
   h->max_a_nnz = keep_max;
@@ -1925,11 +1933,14 @@ int full_replay_impl(oc_spgemm *h, hipStream_t s) {
   const uint64_t m = p.A.rows;
   uint32_t *err = p.err;
   // err[0]: check bits; err[8..9]: bounds of the symbolic overflow list;
-  // err[32]: the row-claim counter of the persistent bin kernels
-  uint32_t *claim = err + 32;
+  // err[32..61]: the row-claim counters of the persistent bin kernels
+  uint32_t *claim = err + 32, *claim_num = claim + Run::kClaimNumeric;
+  static_assert(32 + Run::kClaims <= 64, "the counters fit the plan's check words");
+  auto rows1 = [&](int b) { return p.hoff1[b + 1] - p.hoff1[b]; };
+  auto rows2 = [&](int b) { return p.hoff[b + 1] - p.hoff[b]; };
   const AccArgs a = r.acc();
   const Tables &t = tables();
-  OC_TRY(launch_fill_u32(err, 1, 0u, s));
+  OC_TRY(launch_fill_u32(err, 64, 0u, s));
   OC_TRY(launch_fill_u32(p.ovf, 8, 0u, s));
   // analysis (fixed grid) and the longest A row against the planned one
   OC_TRY(launch_analysis(p.A, p.B, p.ri, p.scal, p.scal + 1, p.ana_tmp, s));
@@ -1946,28 +1957,30 @@ int full_replay_impl(oc_spgemm *h, hipStream_t s) {
   for (int b = 0; b <= 5; ++b) {
     const uint32_t S = t.hash_sym[b];
     OC_TRY(launch_sym_hash(b, a, p.brows1, 0, p.est_symbolic ? S - S / 8 : S, p.nnz, ovf_rows,
-                           p.ovf, s, RowSel{p.boff1 + b, nullptr, claim}));
+                           p.ovf, s, RowSel{p.boff1 + b, nullptr, claim + b, ~0u, rows1(b)}));
   }
   OC_TRY(launch_sym_window(a, p.brows1, 0, p.max_a_nnz, p.nnz, p.win_scratch, s,
-                           RowSel{p.boff1 + 6, err, claim}));
+                           RowSel{p.boff1 + 6, err, claim + 6}));
   for (int b = 8; b <= 13; ++b)
     OC_TRY(launch_sym_dense(b - 7, a, p.brows1, 0, p.nnz, s, nullptr, nullptr,
-                            RowSel{p.boff1 + b, nullptr, claim}));
+                            RowSel{p.boff1 + b, nullptr, claim + b, ~0u, rows1(b)}));
   // rows whose table filled up are recounted by the windowed kernel over
   // the device-side overflow list [0, ovf[0])
   uint32_t *ovf_bounds = err + 8;
   OC_TRY(launch_count_bounds(p.ovf, ovf_bounds, s));
   OC_TRY(launch_sym_window(a, ovf_rows, 0, p.max_a_nnz, p.nnz, p.win_scratch, s,
-                           RowSel{ovf_bounds, err, claim}));
+                           RowSel{ovf_bounds, err, claim + Run::kClaimRecount}));
   // C's offsets, and its capacity against the new nnz
   OC_TRY(launch_scan_u32(p.nnz, (uint64_t *)p.o.off, m, p.scan_tmp, s));
   OC_TRY(launch_check_gt(p.o.off + m, 1, p.cap_nnz, kFullCapacity, err, s));
   // numeric: binning on the exact counts, then every bin persistent
   OC_TRY(launch_binning(p.num_bp, m, p.bor2, const_cast<uint32_t *>(p.brows), p.boff2, p.bin_tmp, s));
   for (int b = 1; b <= 6; ++b)
-    OC_TRY(launch_num_hash(b, a, p.brows, 0, p.o, s, RowSel{p.boff2 + b, err, claim}));
+    OC_TRY(launch_num_hash(b, a, p.brows, 0, p.o, s,
+                           RowSel{p.boff2 + b, err, claim_num + b, ~0u, rows2(b)}));
   for (int b = 7; b <= 12; ++b)
-    OC_TRY(launch_num_dense(b - 7, a, p.brows, 0, p.o, s, RowSel{p.boff2 + b, err, claim}));
+    OC_TRY(launch_num_dense(b - 7, a, p.brows, 0, p.o, s,
+                            RowSel{p.boff2 + b, err, claim_num + b, ~0u, rows2(b)}));
   const uint32_t keep_max = h->max_a_nnz;
   h->max_a_nnz = p.max_a_nnz;
   int rc = r.big_rows(p.brows, 0, p.o, RowSel{p.boff2 + 13, err});
