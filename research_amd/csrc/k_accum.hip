@@ -427,6 +427,181 @@ __device__ __forceinline__ void bin_rows(const uint32_t *__restrict__ bounds, ui
   }
 }
 
+// ==================================================== a row's products, flat
+// Short B rows leave most of a lane group idle and give each lane one load
+// at a time.  Here the products of 64 A entries (a chunk) are numbered by a
+// scan of the B row lengths, and each wave takes blocks of 64 consecutive
+// products, U blocks at a time: every lane has U independent gathers in
+// flight, consecutive lanes read consecutive entries, and no lane idles but
+// in the last block.  `share` waves split a chunk's blocks; BS / 64 / share
+// chunks are in work at once.  B rows longer than `skip` are left out (the
+// caller sweeps them).  f(c, v, ok) takes U columns, B values times the A
+// value (VALS) and whether the lane has a product there, and returns false
+// (the whole wave) to stop.  All lanes of the workgroup call it.
+template <int BS, int U, bool VALS, typename T, typename F>
+__device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uint32_t a1,
+                                             uint32_t share, uint32_t skip, F &&f) {
+  constexpr uint32_t NW = BS / kWave;
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wid =
+      NW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t step = NW / share * kWave, sub = wid % share;
+  uint32_t c0 = a0 + wid / share * kWave;
+  if (c0 >= a1) return;
+  auto add = [](uint32_t x, uint32_t y) { return x + y; };
+  // this chunk's B row bounds and A values, the next chunk's columns
+  uint32_t bs = 0, be = 0, kn = 0;
+  T av = T(0);
+  if (c0 + lane < a1) {
+    const uint32_t k = a.a_ci[c0 + lane];
+    if (VALS) av = a.a_v[c0 + lane];
+    bs = a.b_rp[k];
+    be = a.b_rp[k + 1];
+  }
+  if (c0 + step + lane < a1) kn = a.a_ci[c0 + step + lane];
+  for (;;) {
+    const uint32_t cn = c0 + step;
+    uint32_t bsn = 0, ben = 0;
+    T avn = T(0);
+    if (cn + lane < a1) {
+      bsn = a.b_rp[kn];
+      ben = a.b_rp[kn + 1];
+      if (VALS) avn = a.a_v[cn + lane];
+      if (cn + step + lane < a1) kn = a.a_ci[cn + step + lane];
+    }
+    const uint32_t len = be - bs > skip ? 0u : be - bs;
+    const uint32_t incl = wave_incl_scan(len, 0u, add);
+    const uint32_t ex = incl - len, base = bs - ex;
+    const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    const uint32_t nb = (P + kWave - 1) / kWave, per = (nb + share - 1) / share;
+    const uint32_t b0 = min(nb, sub * per), b1 = min(nb, b0 + per);
+    for (uint32_t b = b0; b < b1; b += U) {
+      uint32_t q[U];
+      T pa[U];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        q[u] = 0;
+        pa[u] = T(0);
+        ok[u] = false;
+        if (b + u < b1) {  // uniform
+          // the A entry of product p: the last non-empty one that starts at
+          // or before it
+          const uint32_t p0 = (b + u) * kWave, p = p0 + lane;
+          ok[u] = p < P;
+          const uint64_t here = __ballot(len != 0 && ex <= p0);
+          uint64_t starts = __ballot(len != 0 && ex > p0 && ex - p0 < kWave);
+          const int first = 63 - __clzll(here);
+          if (starts == 0) {  // one B row gives the whole block
+            q[u] = (uint32_t)__builtin_amdgcn_readlane((int)base, first) + p;
+            if (VALS) pa[u] = __shfl(av, first);
+          } else {
+            int owner = first;
+            if (__popcll(starts) <= 12) {
+              do {
+                const int t = __builtin_ctzll(starts);
+                starts &= starts - 1;
+                const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)ex, t);
+                owner = p >= e ? t : owner;
+              } while (starts);
+            } else {
+              // many short B rows: the last of the ascending starts at or
+              // before p (an empty row's start is that of the row after it)
+              owner = 0;
+#pragma unroll
+              for (int d = 32; d > 0; d >>= 1) {
+                const uint32_t e = __shfl(ex, owner + d);
+                owner = e <= p ? owner + d : owner;
+              }
+            }
+            q[u] = __shfl(base, owner) + p;
+            if (VALS) pa[u] = __shfl(av, owner);
+          }
+        }
+      }
+      uint32_t c[U];
+      T v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        c[u] = 0;
+        v[u] = T(0);
+        if (ok[u]) {
+          c[u] = a.b_ci[q[u]];
+          if (VALS) v[u] = a.b_v[q[u]];
+        }
+      }
+      double pv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) pv[u] = VALS ? product_pz((double)pa[u], (double)v[u]) : 0.0;
+      if (!f(c, pv, ok)) return;
+    }
+    if (cn >= a1) return;
+    c0 = cn;
+    bs = bsn;
+    be = ben;
+    av = avn;
+  }
+}
+
+// Rows whose B rows average fewer entries than this go product by product
+// (for_products), the others by lane groups (for_entries): from about a
+// wave's width on, a group of 64 lanes is as full and finds its entries
+// without a search.  (By products instead of by groups: 99,890 symbolic hash
+// rows of 576 products in B rows of 24, 717 -> 534 us; numeric hash rows of
+// the same product 730 -> 684 us; 131,072 banded rows of 33 x 33, numeric
+// dense, 325 -> 221 us.)
+constexpr uint32_t kFlatAvg = 64;
+
+// Waves per chunk of for_products: enough blocks of 64 products for each (U
+// at a time), and no more chunks at once than the row has.
+template <int BS, int U>
+__device__ __forceinline__ uint32_t flat_share(uint32_t nA, uint32_t avg) {
+  constexpr uint32_t NW = BS / kWave;
+  if constexpr (NW == 1) return 1u;
+  const uint32_t chunks = (nA + kWave - 1) / kWave;
+  uint32_t share = 1;
+  while (share < NW && (2 * share * U <= avg || NW / share > chunks)) share *= 2;
+  return share;
+}
+
+// Lists the A entries whose B row is longer than `longest`; returns how
+// many, or 0 when there are none or more than `cap`.  For chunks that
+// different waves take: a listed row is swept by the whole workgroup.
+template <int BS, typename KA>
+__device__ __forceinline__ uint32_t list_longer(const KA &a, uint32_t a0, uint32_t a1,
+                                                uint32_t longest, uint32_t *count,
+                                                uint32_t *list, uint32_t cap) {
+  for (uint32_t j = a0 + threadIdx.x; j < a1; j += BS) {
+    const uint32_t k = a.a_ci[j];
+    if (a.b_rp[k + 1] - a.b_rp[k] > longest) {
+      const uint32_t idx = atomicAdd(count, 1u);
+      if (idx < cap) list[idx] = j;
+    }
+  }
+  __syncthreads();
+  const uint32_t n = *count;
+  return n <= cap ? n : 0u;
+}
+
+// What a row's flat walk needs: the waves per chunk, the B rows to leave
+// out (longer than skip) and how many of them are listed.
+struct Flat {
+  uint32_t share, skip, listed;
+};
+template <int BS, int U, typename KA>
+__device__ __forceinline__ Flat flat_plan(const KA &a, const RowHead &rh, uint32_t avg,
+                                          uint32_t *count, uint32_t *list, uint32_t cap) {
+  constexpr uint32_t NW = BS / kWave;
+  Flat fl{flat_share<BS, U>(rh.a1 - rh.a0, avg), 0xFFFFFFFFu, 0u};
+  const uint32_t chunks = NW / fl.share;
+  const uint32_t longest = max(512u, 2u * (rh.prod / chunks));
+  if (chunks > 1 && rh.maxb > longest) {
+    fl.listed = list_longer<BS>(a, rh.a0, rh.a1, longest, count, list, cap);
+    if (fl.listed) fl.skip = longest;
+  }
+  return fl;
+}
+
 // ========================================================== symbolic hash
 constexpr uint32_t kSymHeavy = 56;  // listed heavy B rows per row (hdr[8..63])
 constexpr uint32_t kDenseHeavy = 32;  // dense kernels: hdr[32..63], count hdr[4]
@@ -464,11 +639,16 @@ __device__ __forceinline__ void sym_hash_row(KArgs<float> a,
   const uint32_t a0 = rh.a0, a1 = rh.a1;
   const int G = pick_group_lat<8>(a1 - a0, rh.prod, rh.maxb, BS);
   const int ngroups = BS / G, gid = threadIdx.x / G, lig = threadIdx.x % G;
+  const uint32_t avg = a1 > a0 ? rh.prod / (a1 - a0) : 0u;
+  const bool flat = avg < kFlatAvg;
   if (use_bm) {
     auto mark = [&](uint32_t col) {
       const uint32_t c = col - blo;
       atomicOr(&tab[c >> 5], 1u << (c & 31));
     };
+    // (by lane groups also where B rows are short: an OR is one cheap LDS
+    // operation, and finding the products' owners cost more: 634 -> 672 us
+    // on a 128-product batch)
     uint32_t heavy;
     const uint32_t nheavy =
         list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[3], hdr + 8, kSymHeavy, &heavy);
@@ -512,13 +692,16 @@ __device__ __forceinline__ void sym_hash_row(KArgs<float> a,
     if (!ovf) probe(c, hash_slot(c, S), 0);
   };
   // eight keys: first probes issued together, collisions probed on
-  auto insert8 = [&](const uint32_t (&c)[8]) {
+  auto insert8_if = [&](const uint32_t (&c)[8], const bool (&ok)[8]) {
     if (ovf) return;
     uint32_t sl[8], old[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) sl[u] = hash_slot(c[u], S);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) old[u] = atomicCAS(&tab[sl[u]], kEmpty, c[u]);
+    for (int u = 0; u < 8; ++u) {
+      old[u] = c[u];  // nothing to insert
+      if (ok[u]) old[u] = atomicCAS(&tab[sl[u]], kEmpty, c[u]);
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (old[u] == kEmpty) {
@@ -529,19 +712,39 @@ __device__ __forceinline__ void sym_hash_row(KArgs<float> a,
       }
     }
   };
-  uint32_t heavy;
-  const uint32_t nheavy =
-      list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[3], hdr + 8, kSymHeavy, &heavy);
-  for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
-              [&](uint32_t, uint32_t bs, uint32_t be) {
-                if (track && lds_load(&hdr[0]) > limit) {  // past the load limit
-                  ovf = true;
-                  return false;
-                }
-                if (!(nheavy && be - bs > heavy))  // listed: swept below
-                  seg_cols_batch<8>(bs, be, lig, G, a.b_ci, insert8, insert);
-                return !ovf;
-              });
+  auto insert8 = [&](const uint32_t (&c)[8]) {
+    const bool all[8] = {true, true, true, true, true, true, true, true};
+    insert8_if(c, all);
+  };
+  uint32_t nheavy;
+  if (flat) {
+    const Flat fl = flat_plan<BS, 8>(a, rh, avg, &hdr[3], hdr + 8, kSymHeavy);
+    nheavy = fl.listed;
+    for_products<BS, 8, false>(
+        a, a0, a1, fl.share, fl.skip,
+        [&](const uint32_t (&c)[8], const double (&)[8], const bool (&ok)[8]) {
+          if (track && __builtin_amdgcn_readfirstlane(lds_load(&hdr[0])) > limit) {
+            ovf = true;  // past the load limit
+            return false;
+          }
+          insert8_if(c, ok);
+          return true;
+        });
+  } else {
+    uint32_t heavy;
+    nheavy =
+        list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[3], hdr + 8, kSymHeavy, &heavy);
+    for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
+                [&](uint32_t, uint32_t bs, uint32_t be) {
+                  if (track && lds_load(&hdr[0]) > limit) {  // past the load limit
+                    ovf = true;
+                    return false;
+                  }
+                  if (!(nheavy && be - bs > heavy))  // listed: swept below
+                    seg_cols_batch<8>(bs, be, lig, G, a.b_ci, insert8, insert);
+                  return !ovf;
+                });
+  }
   __syncthreads();
   for (uint32_t h = 0; h < nheavy && !ovf; ++h) {
     if (track && lds_load(&hdr[0]) > limit) {
@@ -732,15 +935,19 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
     if (!ovf) probe(c, pv, hash_slot(c, S), 0);
   };
   // four products: first probes issued together, collisions probed on
-  auto insert4 = [&](const uint32_t (&c)[4], const double (&pv)[4]) {
+  auto insert4_if = [&](const uint32_t (&c)[4], const double (&pv)[4], const bool (&ok)[4]) {
     if (ovf) return;
     uint32_t sl[4], old[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) sl[u] = hash_slot(c[u], S);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) old[u] = atomicCAS(&keys[sl[u]], kEmpty, c[u]);
+    for (int u = 0; u < 4; ++u) {
+      old[u] = 0;
+      if (ok[u]) old[u] = atomicCAS(&keys[sl[u]], kEmpty, c[u]);
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      if (!ok[u]) continue;
       if (old[u] == kEmpty || old[u] == c[u]) {
         if (EST && old[u] == kEmpty) atomicAdd(&hdr[0], 1u);
         lds_add_f64(&vals[sl[u]], pv[u]);
@@ -749,20 +956,41 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
       }
     }
   };
-  uint32_t heavy;  // heavy B rows listed and swept by the whole workgroup
-  const uint32_t nheavy =
-      list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[3], hdr + 8, kSymHeavy, &heavy);
-  for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
-              [&](uint32_t j, uint32_t bs, uint32_t be) {
-                if (EST && lds_load(&hdr[0]) > limit) {  // more keys than the capacity
-                  ovf = true;
-                  return false;
-                }
-                if (!(nheavy && be - bs > heavy))  // listed: swept below
-                  seg_vals_batch<4>(bs, be, lig, G, (double)a.a_v[j], a.b_ci, a.b_v, insert4,
-                                    insert);
-                return !ovf;
-              });
+  auto insert4 = [&](const uint32_t (&c)[4], const double (&pv)[4]) {
+    const bool all[4] = {true, true, true, true};
+    insert4_if(c, pv, all);
+  };
+  uint32_t nheavy;  // heavy B rows listed and swept by the whole workgroup
+  const uint32_t avg = a1 > a0 ? rh.prod / (a1 - a0) : 0u;
+  if (avg < kFlatAvg) {
+    const Flat fl = flat_plan<BS, 4>(a, rh, avg, &hdr[3], hdr + 8, kSymHeavy);
+    nheavy = fl.listed;
+    for_products<BS, 4, true>(
+        a, a0, a1, fl.share, fl.skip,
+        [&](const uint32_t (&c)[4], const double (&pv)[4], const bool (&ok)[4]) {
+          if (EST && __builtin_amdgcn_readfirstlane(lds_load(&hdr[0])) > limit) {
+            ovf = true;  // more keys than the capacity
+            return false;
+          }
+          insert4_if(c, pv, ok);
+          return true;
+        });
+  } else {
+    uint32_t heavy;
+    nheavy =
+        list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[3], hdr + 8, kSymHeavy, &heavy);
+    for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
+                [&](uint32_t j, uint32_t bs, uint32_t be) {
+                  if (EST && lds_load(&hdr[0]) > limit) {  // more keys than the capacity
+                    ovf = true;
+                    return false;
+                  }
+                  if (!(nheavy && be - bs > heavy))  // listed: swept below
+                    seg_vals_batch<4>(bs, be, lig, G, (double)a.a_v[j], a.b_ci, a.b_v, insert4,
+                                      insert);
+                  return !ovf;
+                });
+  }
   __syncthreads();
   for (uint32_t h = 0; h < nheavy && !ovf; ++h) {
     if (EST && lds_load(&hdr[0]) > limit) {
@@ -984,15 +1212,30 @@ __device__ __forceinline__ void num_dense_row(KArgs<T> a,
   const int G = pick_group(a1 - a0, rh.prod, rh.maxb, BS);
   const int ngroups = BS / G, gid = threadIdx.x / G, lig = threadIdx.x % G;
   auto add = [&](uint32_t col, double pv) { lds_add_f64(&vals[col - lo], pv); };
-  uint32_t heavy;  // heavy B rows listed and swept by the whole workgroup
-  const uint32_t nheavy =
-      list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[4], hdr + 32, kDenseHeavy, &heavy);
-  for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
-              [&](uint32_t j, uint32_t bs, uint32_t be) {
-                if (!(nheavy && be - bs > heavy))
-                  seg_vals<4>(bs, be, lig, G, (double)a.a_v[j], a.b_ci, a.b_v, add);
-                return true;
-              });
+  uint32_t nheavy;  // heavy B rows listed and swept by the whole workgroup
+  const uint32_t avg = rh.prod / (a1 - a0);
+  if (avg < kFlatAvg) {
+    const Flat fl = flat_plan<BS, 4>(a, rh, avg, &hdr[4], hdr + 32, kDenseHeavy);
+    nheavy = fl.listed;
+    for_products<BS, 4, true>(a, a0, a1, fl.share, fl.skip,
+                              [&](const uint32_t (&c)[4], const double (&pv)[4],
+                                  const bool (&ok)[4]) {
+#pragma unroll
+                                for (int u = 0; u < 4; ++u)
+                                  if (ok[u]) add(c[u], pv[u]);
+                                return true;
+                              });
+  } else {
+    uint32_t heavy;
+    nheavy =
+        list_heavy(a, rh, a0, a1, G, gid, ngroups, lig, &hdr[4], hdr + 32, kDenseHeavy, &heavy);
+    for_entries(a, a0, a1, (uint32_t)gid, (uint32_t)ngroups,
+                [&](uint32_t j, uint32_t bs, uint32_t be) {
+                  if (!(nheavy && be - bs > heavy))
+                    seg_vals<4>(bs, be, lig, G, (double)a.a_v[j], a.b_ci, a.b_v, add);
+                  return true;
+                });
+  }
   for (uint32_t h = 0; h < nheavy; ++h) {
     const uint32_t j = hdr[32 + h];
     const uint32_t k = a.a_ci[j];
