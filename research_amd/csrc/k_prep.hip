@@ -138,7 +138,15 @@ constexpr int kLongBlock = 256;
 
 __global__ __launch_bounds__(256) void k_brow_info(const uint32_t *__restrict__ b_rp,
                                                    const uint32_t *__restrict__ b_ci,
-                                                   uint32_t b_rows, uint4 *__restrict__ info) {
+                                                   uint32_t b_rows, uint4 *__restrict__ info,
+                                                   uint32_t *z0, uint32_t *z1, uint32_t *z2) {
+  // the counters of the kernels that follow, cleared here rather than by a
+  // launch or a memset node of their own (capture-safe)
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (z0) *z0 = 0;
+    if (z1) *z1 = 0;
+    if (z2) *z2 = 0;
+  }
   for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < b_rows; k += gridDim.x * 256) {
     const uint32_t bs = b_rp[k], be = b_rp[k + 1];
     uint4 v = make_uint4(0u, 0xFFFFFFFFu, 0u, 0u);
@@ -379,12 +387,11 @@ int launch_analysis(const DevCsr &A, const DevCsr &B, const RowInfo &ri,
   uint4 *info = (uint4 *)temp;
   uint32_t *long_count = (uint32_t *)(info + B.rows + 1);
   uint32_t *long_rows = long_count + 64;
-  // counters cleared by a kernel, not memset nodes (capture-safe)
-  hipLaunchKernelGGL(k_zero3, dim3(1), dim3(64), 0, s, long_count, max_a_nnz, max_products);
+  hipLaunchKernelGGL(k_brow_info,
+                     dim3(std::max<uint64_t>(1, std::min<uint64_t>(cdiv(B.rows, 256), 1u << 20))),
+                     dim3(256), 0, s, B.rp, B.ci, (uint32_t)B.rows, info, long_count, max_a_nnz,
+                     max_products);
   LAUNCH_CHECK();
-  if (B.rows)
-    hipLaunchKernelGGL(k_brow_info, dim3(std::min<uint64_t>(cdiv(B.rows, 256), 1u << 20)),
-                       dim3(256), 0, s, B.rp, B.ci, (uint32_t)B.rows, info);
   const double avg = (double)A.nnz / (double)A.rows;
   const uint32_t rows = (uint32_t)A.rows;
   // at most the resident workgroups (two per CU); lanes for about half of the
@@ -409,6 +416,32 @@ int launch_analysis(const DevCsr &A, const DevCsr &B, const RowInfo &ri,
                      long_rows, long_count);
   LAUNCH_CHECK();
   if (own) HIP_TRY(hipFreeAsync(own, s));
+  return OC_OK;
+}
+
+// ------------------------------------------------- small results to the host
+// Copies a few device words into a pinned host page and then sets the page's
+// flag, on which the host spins.  A copy into pageable memory and a stream
+// synchronisation took 12 us more for each value the host waits for.
+__global__ __launch_bounds__(1024) void k_publish(PublishArgs pa, uint32_t *dst, uint32_t *flag,
+                                                  uint32_t seq) {
+  uint32_t at = 0;
+  for (int k = 0; k < PublishArgs::kMax; ++k) {
+    for (uint32_t i = threadIdx.x; i < pa.words[k]; i += blockDim.x) dst[at + i] = pa.src[k][i];
+    at += pa.words[k];
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int launch_publish(const PublishArgs &pa, uint32_t *dst, uint32_t *flag, uint32_t seq,
+                   hipStream_t s) {
+  uint32_t most = 0;
+  for (int k = 0; k < PublishArgs::kMax; ++k) most = std::max(most, pa.words[k]);
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(most > 64 ? 1024 : 64), 0, s, pa, dst, flag, seq);
+  LAUNCH_CHECK();
   return OC_OK;
 }
 

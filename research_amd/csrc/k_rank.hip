@@ -617,48 +617,46 @@ uint32_t rank1_wide_log(uint32_t bs) {
 
 // ------------------------------------------------------ stored row bitmaps
 // Rows of the dense symbolic bins with at least min_products products get
-// a bitmap region: n4 = ((right - (left & ~127)) >> 7) + 1 uint4 groups.
-__global__ __launch_bounds__(256) void k_bm_sizes(const uint32_t *__restrict__ rows, uint32_t n,
+// a bitmap region: n4 = ((right - (left & ~127)) >> 7) + 1 uint4 groups, in
+// row order (the bins' sizes need not be known on the host).
+__global__ __launch_bounds__(256) void k_bm_sizes(const uint8_t *__restrict__ bin_of_row,
+                                                  int bin_lo, int bin_hi, uint32_t m,
                                                   const uint32_t *__restrict__ products,
                                                   const uint32_t *__restrict__ left,
                                                   const uint32_t *__restrict__ right,
                                                   uint32_t min_products, uint32_t *__restrict__ sz) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t r = rows[i];
-  const uint32_t l = left[r], h = right[r];
-  sz[i] = (products[r] >= min_products && h >= l) ? ((h - (l & ~127u)) >> 7) + 1 : 0u;
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= m) return;
+  const int bin = bin_of_row[r];
+  uint32_t n4 = 0;
+  if (bin >= bin_lo && bin < bin_hi && products[r] >= min_products) {
+    const uint32_t l = left[r], h = right[r];
+    if (h >= l) n4 = ((h - (l & ~127u)) >> 7) + 1;
+  }
+  sz[r] = n4;
 }
 
-__global__ __launch_bounds__(256) void k_bm_fill(uint64_t *__restrict__ bmoff, uint64_t m) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    bmoff[i] = ~0ull;
+__global__ __launch_bounds__(256) void k_bm_mark(const uint32_t *__restrict__ sz, uint32_t m,
+                                                 uint64_t *__restrict__ bmoff) {
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < m && sz[r] == 0) bmoff[r] = ~0ull;
 }
 
-__global__ __launch_bounds__(256) void k_bm_scatter(const uint32_t *__restrict__ rows, uint32_t n,
-                                                    const uint32_t *__restrict__ sz,
-                                                    const uint64_t *__restrict__ offs,
-                                                    uint64_t *__restrict__ bmoff) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (sz[i]) bmoff[rows[i]] = offs[i];
-}
-
-int launch_bitmap_offsets(const uint32_t *rows, uint32_t n, uint64_t m,
+int launch_bitmap_offsets(const uint8_t *bin_of_row, int bin_lo, int bin_hi, uint64_t m,
                           const uint32_t *products, const uint32_t *left,
                           const uint32_t *right, uint32_t min_products, uint32_t *sz,
-                          uint64_t *offs, void *scan_tmp, uint64_t *bmoff, hipStream_t s) {
-  hipLaunchKernelGGL(k_bm_fill, dim3((uint32_t)std::min<uint64_t>(cdiv(m, 256), 4096)), dim3(256),
-                     0, s, bmoff, m);
-  LAUNCH_CHECK();
-  if (n == 0) return OC_OK;
-  hipLaunchKernelGGL(k_bm_sizes, dim3(cdiv(n, 256)), dim3(256), 0, s, rows, n, products, left,
-                     right, min_products, sz);
-  LAUNCH_CHECK();
-  OC_TRY(launch_scan_u32(sz, offs, n, scan_tmp, s));
-  hipLaunchKernelGGL(k_bm_scatter, dim3(cdiv(n, 256)), dim3(256), 0, s, rows, n, sz, offs, bmoff);
-  LAUNCH_CHECK();
+                          void *scan_tmp, uint64_t *bmoff, hipStream_t s) {
+  if (m) {
+    hipLaunchKernelGGL(k_bm_sizes, dim3(cdiv(m, 256)), dim3(256), 0, s, bin_of_row, bin_lo,
+                       bin_hi, (uint32_t)m, products, left, right, min_products, sz);
+    LAUNCH_CHECK();
+  }
+  OC_TRY(launch_scan_u32(sz, bmoff, m, scan_tmp, s));
+  if (m) {
+    hipLaunchKernelGGL(k_bm_mark, dim3(cdiv(m, 256)), dim3(256), 0, s, (const uint32_t *)sz,
+                       (uint32_t)m, bmoff);
+    LAUNCH_CHECK();
+  }
   return OC_OK;
 }
 

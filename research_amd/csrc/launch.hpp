@@ -69,6 +69,15 @@ int launch_analysis(const DevCsr &A, const DevCsr &B, const RowInfo &ri,
 int launch_check_gt(const void *x, int is64, uint64_t limit, uint32_t bit, uint32_t *err,
                     hipStream_t s);
 int launch_fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t s);
+// Device words copied one after another to dst (pinned host memory), then
+// *flag = seq.
+struct PublishArgs {
+  static constexpr int kMax = 3;
+  const uint32_t *src[kMax] = {nullptr, nullptr, nullptr};
+  uint32_t words[kMax] = {0, 0, 0};
+};
+int launch_publish(const PublishArgs &pa, uint32_t *dst, uint32_t *flag, uint32_t seq,
+                   hipStream_t s);
 // bounds = {0, *count}: the row range of a device-counted list
 int launch_count_bounds(const uint32_t *count, uint32_t *bounds, hipStream_t s);
 size_t scan_temp_bytes(uint64_t n);
@@ -250,13 +259,13 @@ int launch_num_rank1(const AccArgs &a, const uint32_t *rows, uint32_t nrows, uin
                      const NumOut &o, void *scratch, hipStream_t s,
                      const RowSel &sel = RowSel{}, uint32_t bs = 1024,
                      const R1Pieces &pc = R1Pieces{});
-// Stored-bitmap offsets (uint4 units) for the listed rows with at least
-// min_products products; bmoff[0..m) = ~0 elsewhere; offs[n] = total.
-// sz: n u32, offs: n + 1 u64, scan_tmp: scan_temp_bytes(n).
-int launch_bitmap_offsets(const uint32_t *rows, uint32_t n, uint64_t m,
+// Stored-bitmap offsets (uint4 units) of the rows in the bins [bin_lo,
+// bin_hi) with at least min_products products; bmoff[0..m) = ~0 elsewhere,
+// bmoff[m] = total.  sz: m u32, scan_tmp: scan_temp_bytes(m).
+int launch_bitmap_offsets(const uint8_t *bin_of_row, int bin_lo, int bin_hi, uint64_t m,
                           const uint32_t *products, const uint32_t *left,
                           const uint32_t *right, uint32_t min_products, uint32_t *sz,
-                          uint64_t *offs, void *scan_tmp, uint64_t *bmoff, hipStream_t s);
+                          void *scan_tmp, uint64_t *bmoff, hipStream_t s);
 // Ultra-sparse expand-sort-compress for all rows with products <= esc_n.
 int launch_esc(int esc_n, const AccArgs &a, const NumOut &o, hipStream_t s);
 

@@ -8,9 +8,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <map>
+#include <mutex>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -142,31 +145,87 @@ struct Arena {
 };
 
 // Stream-ordered timestamps; the time between two marks is charged to the
-// later mark's stage.  Resolved once the stream has drained.
+// later mark's stage.  Resolved once the stream has drained.  The events
+// belong to the handle and are used again by its next run (creating and
+// destroying them cost 0.8 us each); each record still takes the stream
+// about 2.4 us, so a stage in which the run issues nothing is marked none():
+// zero, without an event.
 struct Marks {
   hipStream_t s;
-  std::vector<std::pair<std::string, hipEvent_t>> ev;
+  std::vector<hipEvent_t> &pool;
+  std::vector<const char *> name;  // of pool[i]
+  std::vector<const char *> empty;
   bool enabled = true;
-  explicit Marks(hipStream_t st) : s(st) {}
-  ~Marks() {
-    for (auto &p : ev) (void)hipEventDestroy(p.second);
-  }
-  void mark(const char *name) {
+  Marks(hipStream_t st, std::vector<hipEvent_t> &p) : s(st), pool(p) {}
+  void mark(const char *n) {
     if (!enabled) return;
-    hipEvent_t e;
-    if (hipEventCreate(&e) != hipSuccess) return;
-    (void)hipEventRecord(e, s);
-    ev.emplace_back(name, e);
+    if (name.size() == pool.size()) {
+      hipEvent_t e;
+      if (hipEventCreate(&e) != hipSuccess) return;
+      pool.push_back(e);
+    }
+    (void)hipEventRecord(pool[name.size()], s);
+    name.push_back(n);
+  }
+  void none(const char *n) {
+    if (enabled) empty.push_back(n);
   }
   void resolve(std::map<std::string, double> &out, double &total) {
     total = 0;
-    for (size_t i = 1; i < ev.size(); ++i) {
+    for (const char *n : empty) out[n] += 0.0;
+    for (size_t i = 1; i < name.size(); ++i) {
       float ms = 0;
-      if (hipEventElapsedTime(&ms, ev[i - 1].second, ev[i].second) == hipSuccess) {
-        out[ev[i].first] += ms;
+      if (hipEventElapsedTime(&ms, pool[i - 1], pool[i]) == hipSuccess) {
+        out[name[i]] += ms;
         total += ms;
       }
     }
+  }
+};
+
+// A pinned host page that kernels write small results to (k_publish): word
+// 0 is the flag, the data start at word 16.
+// A handle takes its page on its first run and gives it back when it is
+// destroyed, with no work in flight; up to kIdle pages wait for the next
+// handles (allocating and freeing one costs about 100 us).
+struct HostPage {
+  static constexpr uint32_t kWords = 24 * 1024, kData = 16, kIdle = 16;
+  uint32_t *p = nullptr, seq = 0;
+  struct Idle {
+    std::mutex mu;
+    std::vector<uint32_t *> pages;
+  };
+  static Idle &idle() {
+    static Idle *i = new Idle();  // never destroyed: freed at process exit
+    return *i;
+  }
+  hipError_t take() {
+    if (p) return hipSuccess;
+    {
+      Idle &i = idle();
+      std::lock_guard<std::mutex> lk(i.mu);
+      if (!i.pages.empty()) {
+        p = i.pages.back();
+        i.pages.pop_back();
+      }
+    }
+    if (!p) {
+      const hipError_t e = hipHostMalloc((void **)&p, kWords * 4, hipHostMallocPortable);
+      if (e != hipSuccess) {
+        p = nullptr;
+        return e;
+      }
+    }
+    p[0] = seq = 0;
+    return hipSuccess;
+  }
+  void give() {
+    if (!p) return;
+    Idle &i = idle();
+    std::lock_guard<std::mutex> lk(i.mu);
+    if (i.pages.size() < kIdle) i.pages.push_back(p);
+    else (void)hipHostFree(p);
+    p = nullptr;
   }
 };
 
@@ -302,7 +361,12 @@ struct oc_spgemm {
     plan = Plan();
   }
   ChunkStore mem;  // temporaries of the runs (see ChunkStore)
+  std::vector<hipEvent_t> events;  // of Marks
+  HostPage page;
+  size_t dev_bytes = 0;  // the device's memory (set by the first run)
   ~oc_spgemm() {
+    for (hipEvent_t e : events) (void)hipEventDestroy(e);
+    page.give();
     if (!mem.chunks.empty()) (void)hipDeviceSynchronize();
     mem.drop();
     drop_plan();
@@ -449,7 +513,7 @@ struct Run {
   }
   Run(oc_spgemm *hh, hipStream_t st, oc_csr *cc)
       : h(hh), tscope(hh->custom_shapes ? &hh->shapes : nullptr), c(hh->cfg), s(st),
-        ar(&hh->mem), mk(st), C(cc) {}
+        ar(&hh->mem), mk(st, hh->events), C(cc) {}
 
   AccArgs acc() const {
     AccArgs a;
@@ -462,15 +526,65 @@ struct Run {
     return a;
   }
 
-  // the row-claim counters of the persistent bin launches, one each
+  // ------------------------------------------------ values for the host
+  // publish() queues a copy of a few device words to the handle's pinned
+  // page; await() waits for the latest one and returns them.  The wait spins
+  // on the page's flag, and after 200 us synchronises with the stream
+  // instead, which also reports a failed launch.
+  struct Words {
+    const void *dev;
+    uint32_t n;
+  };
+  int publish(std::initializer_list<Words> w) {
+    HostPage &pg = h->page;
+    HIP_TRY(pg.take());
+    PublishArgs pa;
+    int k = 0;
+    uint32_t total = 0;
+    for (const Words &x : w) {
+      OC_REQUIRE(k < PublishArgs::kMax, "internal: too many values for one host read");
+      pa.src[k] = (const uint32_t *)x.dev;
+      pa.words[k++] = x.n;
+      total += x.n;
+    }
+    OC_REQUIRE(total <= HostPage::kWords - HostPage::kData, "internal: a host read of %u words",
+               total);
+    return launch_publish(pa, pg.p + HostPage::kData, pg.p, ++pg.seq, s);
+  }
+  int await(const uint32_t **out) {
+    HostPage &pg = h->page;
+    *out = pg.p + HostPage::kData;
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int i = 0; i < 64; ++i) {
+        if (__atomic_load_n(pg.p, __ATOMIC_ACQUIRE) == pg.seq) return OC_OK;
+        __builtin_ia32_pause();
+      }
+    } while (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200));
+    HIP_TRY(hipStreamSynchronize(s));
+    OC_REQUIRE(__atomic_load_n(pg.p, __ATOMIC_ACQUIRE) == pg.seq,
+               "internal: a host read did not complete");
+    return OC_OK;
+  }
+  int fetch(std::initializer_list<Words> w, const uint32_t **out) {
+    OC_TRY(publish(w));
+    return await(out);
+  }
+  static uint64_t u64_at(const uint32_t *p) { return (uint64_t)p[0] | (uint64_t)p[1] << 32; }
+
+  // Counters of a run, cleared by one launch: [0..7] overflow counts, from
+  // kCtlClaims on the row-claim counters of the persistent bin launches, one
+  // each
   // (symbolic bin b: b, the recount of overflow rows: 14, numeric bin b:
-  // 16 + b), all cleared by one launch before the first of them
+  // 16 + b).  The overflow list follows at kCtlWords.
   static constexpr uint32_t kClaims = 30, kClaimRecount = 14, kClaimNumeric = 16;
+  static constexpr uint32_t kCtlClaims = 16, kCtlWords = 64;
   uint32_t *claim_ctr = nullptr;
-  int claims() {
-    if (claim_ctr) return OC_OK;
-    OC_TRY(ar.get(&claim_ctr, 64));
-    return launch_fill_u32(claim_ctr, kClaims, 0u, s);
+  int counters(uint32_t **ovf, uint32_t **ovf_rows) {
+    OC_TRY(ar.get(ovf, A.rows + kCtlWords));
+    *ovf_rows = *ovf + kCtlWords;
+    claim_ctr = *ovf + kCtlClaims;
+    return launch_fill_u32(*ovf, kCtlWords, 0u, s);
   }
 
   int window_scratch() {
@@ -517,33 +631,31 @@ struct Run {
     return OC_OK;
   }
 
-  // Row bitmaps of the windowed and dense symbolic bins (rows with at
+  // Row bitmaps of the windowed and dense symbolic bins 6..13 (rows with at
   // least kBitmapMinProducts products), stored by the symbolic pass for the
-  // one-gather rank tiles of the numeric pass.  The bins' rows are
-  // [hoff[6], hoff[14]) (bin 7 is never used).  Skipped for block-diagonal
+  // one-gather rank tiles of the numeric pass.  Skipped for block-diagonal
   // batches and when the bitmaps would take more than a fifth of the device.
-  int row_bitmaps(const uint32_t *brows, const uint32_t *hoff) {
-    constexpr uint32_t kBitmapMinProducts = 2048;
+  // Their offsets are queued with the binning, whose bin sizes the host reads
+  // together with the bitmaps' size.
+  static constexpr uint32_t kBitmapMinProducts = 2048;
+  uint64_t *bmoff_all = nullptr;
+  int bitmap_offsets(const uint8_t *bor) {
     h->bitmap_bytes = 0;
     const bool blocks = h->b_block_base != nullptr && h->b_block_rp == (const void *)B.rp;
-    if (h->cfg.use_tiled_numeric != 3 || blocks || hoff[14] <= hoff[6]) return OC_OK;
-    const uint32_t nd = hoff[14] - hoff[6];
-    uint64_t *bmoff, *offs;
+    if (h->cfg.use_tiled_numeric != 3 || blocks || h->max_products < kBitmapMinProducts)
+      return OC_OK;
     uint32_t *sz;
-    OC_TRY(ar.get(&bmoff, A.rows));
-    OC_TRY(ar.get(&sz, nd));
-    OC_TRY(ar.get(&offs, (uint64_t)nd + 1));
-    OC_TRY(launch_bitmap_offsets(brows + hoff[6], nd, A.rows, ri.products, ri.left, ri.right,
-                                 kBitmapMinProducts, sz, offs, scan_tmp, bmoff, s));
-    uint64_t n4 = 0;
-    OC_TRY(readback(&n4, offs + nd, 1, s));
-    size_t fr = 0, tot = 0;
-    HIP_TRY(hipMemGetInfo(&fr, &tot));
-    if (n4 == 0 || (double)n4 * 16 > 0.2 * (double)tot) return OC_OK;
+    OC_TRY(ar.get(&bmoff_all, A.rows + 1));
+    OC_TRY(ar.get(&sz, A.rows));
+    return launch_bitmap_offsets(bor, 6, 14, A.rows, ri.products, ri.left, ri.right,
+                                 kBitmapMinProducts, sz, scan_tmp, bmoff_all, s);
+  }
+  int row_bitmaps(uint64_t n4) {
+    if (n4 == 0 || (double)n4 * 16 > 0.2 * (double)h->dev_bytes) return OC_OK;
     uint8_t *bm;
     OC_TRY(ar.get(&bm, n4 * 16));
     row_bm = bm;
-    row_bmoff = bmoff;
+    row_bmoff = bmoff_all;
     h->bitmap_bytes = n4 * 16;
     return OC_OK;
   }
@@ -599,21 +711,23 @@ struct Run {
     return launch_num_window(acc(), rows, n, h->max_a_nnz, o, win_scratch, s, sel);
   }
 
-  // C: u64 offsets (rows+1) from per-row counts, then cols/values.
-  int alloc_c_from_counts(const uint32_t *nnz) {
+  // C: u64 offsets (rows+1) from per-row counts, then (once the host has
+  // read offsets[rows]) cols/values.
+  int c_offsets(const uint32_t *nnz) {
     const uint64_t m = A.rows;
-    std::memset(C, 0, sizeof(*C));
-    C->rows = m;
-    C->cols = B.cols;
-    C->vtype = A.vtype;
-    C->off_bytes = 8;
-    C->on_device = 1;
-    C->owned = 3;  // output cache (out_alloc)
-    OC_TRY(out_alloc(&C->row_offsets, (m + 1) * 8));
-    OC_TRY(launch_scan_u32(nnz, (uint64_t *)C->row_offsets, m, scan_tmp, s));
-    mk.mark("epilogue_scan");
-    uint64_t nnzc = 0;
-    OC_TRY(readback(&nnzc, (const uint64_t *)C->row_offsets + m, 1, s));
+    if (!C->row_offsets) {
+      C->rows = m;
+      C->cols = B.cols;
+      C->vtype = A.vtype;
+      C->off_bytes = 8;
+      C->on_device = 1;
+      C->owned = 3;  // output cache (out_alloc)
+      OC_TRY(out_alloc(&C->row_offsets, (m + 1) * 8));
+    }
+    return launch_scan_u32(nnz, (uint64_t *)C->row_offsets, m, scan_tmp, s);
+  }
+  Words c_nnz() const { return Words{(const uint64_t *)C->row_offsets + A.rows, 2}; }
+  int c_entries(uint64_t nnzc) {
     C->nnz = nnzc;
     OC_TRY(out_alloc((void **)&C->col_ids, std::max<uint64_t>(nnzc, 1) * 4));
     OC_TRY(out_alloc(&C->values, std::max<uint64_t>(nnzc, 1) * vsize(A.vtype)));
@@ -621,8 +735,8 @@ struct Run {
     return OC_OK;
   }
 
-  int binning(const BinParams &bp, uint8_t **bor, uint32_t **brows,
-              uint32_t **boff, uint32_t *hoff) {
+  // Queues the binning; the caller reads the bin offsets (boff).
+  int queue_binning(const BinParams &bp, uint8_t **bor, uint32_t **brows, uint32_t **boff) {
     const uint64_t m = A.rows;
     if (!*bor) {
       OC_TRY(ar.get(bor, m));
@@ -632,9 +746,7 @@ struct Run {
     uint8_t *tmp;
     OC_TRY(ar.get(&tmp, bin_temp_bytes(m)));
     bin_tmp = tmp;
-    OC_TRY(launch_binning(bp, m, *bor, *brows, *boff, tmp, s));
-    OC_TRY(readback(hoff, *boff, kBinSlots + 1, s));
-    return OC_OK;
+    return launch_binning(bp, m, *bor, *brows, *boff, tmp, s);
   }
 
   // Select the long rows for the band kernels and build their tables.
@@ -698,7 +810,10 @@ struct Run {
   int numeric_bins(const uint32_t *brows, const uint32_t *hoff, const NumOut &o,
                    bool window_bin13, const uint32_t *boff = nullptr) {
     const AccArgs a = acc();
-    if (boff) OC_TRY(claims());
+    auto stage = [&](const char *name, bool work) {
+      if (work) mk.mark(name);
+      else mk.none(name);
+    };
     for (int b = 0; b <= 6; ++b) {
       const uint32_t n = hoff[b + 1] - hoff[b];
       if (!n) continue;
@@ -713,7 +828,7 @@ struct Run {
         OC_TRY(launch_num_hash(b, a, brows + hoff[b], n, o, s));
     }
     fam("num_hash", "numeric_hash", true, brows + hoff[1], hoff[7] - hoff[1]);
-    mk.mark("numeric_hash");
+    stage("numeric_hash", hoff[7] > hoff[0]);
     for (int b = 7; b <= 12; ++b) {
       const uint32_t n = hoff[b + 1] - hoff[b];
       if (!n) continue;
@@ -724,14 +839,14 @@ struct Run {
         OC_TRY(launch_num_dense(b - 7, a, brows + hoff[b], n, o, s));
     }
     fam("num_dense", "numeric_dense", true, brows + hoff[7], hoff[13] - hoff[7]);
-    mk.mark("numeric_dense");
+    stage("numeric_dense", hoff[13] > hoff[7]);
     if (window_bin13) {
       const uint32_t n = hoff[14] - hoff[13];
+      mk.none("numeric_tile_starts");  // tiles() marks it when it builds them
       if (n) OC_TRY(tiles());
-      mk.mark("numeric_tile_starts");
       OC_TRY(big_rows(brows + hoff[13], n, o));
       fam("num_window", "numeric_window", true, brows + hoff[13], n);
-      mk.mark("numeric_window");
+      stage("numeric_window", n != 0);
     }
     return OC_OK;
   }
@@ -743,7 +858,14 @@ struct Run {
   int run_fat();
   int run_usparse();
   int run_precise();
+  int finish_precise();
   int run_est();
+  // rows the precise numeric kernels listed, read once the stream has drained
+  struct Recount {
+    bool pending = false;
+    uint32_t *rows = nullptr;
+    NumOut o{};
+  } recount;
 };
 
 int Run::prologue_and_analysis() {
@@ -769,7 +891,7 @@ int Run::prologue_and_analysis() {
   const bool largest = !((uint32_t)bits_needed(B.cols ? B.cols - 1 : 0) > idx_bits6 ||
                          !c.use_hybrid_accumulator) &&
                        B.cols > (uint64_t)c.numeric_hybrid_hash_kernel_row_length_threshold;
-  mk.mark("prologue");
+  mk.none("prologue");
   uint8_t *atmp;
   OC_TRY(ar.get(&atmp, analysis_temp_bytes(m, A.nnz, B.rows)));
   OC_TRY(launch_analysis(A, B, ri, scal, scal + 1, atmp, s));
@@ -780,11 +902,11 @@ int Run::prologue_and_analysis() {
   mk.mark("analysis_product_calc");
   OC_TRY(launch_scan_u32(ri.products, psum_prod, m, scan_tmp, s));
   mk.mark("analysis_reduce");
-  uint32_t sc[2];
-  OC_TRY(readback(sc, scal, 2, s));
-  OC_TRY(readback(&h->total_products, psum_prod + m, 1, s));
-  h->max_a_nnz = sc[0];
-  h->max_products = sc[1];
+  const uint32_t *w;
+  OC_TRY(fetch({{scal, 2}, {psum_prod + m, 2}}, &w));
+  h->max_a_nnz = w[0];
+  h->max_products = w[1];
+  h->total_products = u64_at(w + 2);
   mk.mark("analysis_mem_cpy");
   decide_analysis(c, *h, h->d);
   h->d.hash_largest = largest;
@@ -795,7 +917,7 @@ int Run::sampling() {
   Decision &d = h->d;
   const int P = 1 << d.log_p;
   OC_TRY(ar.get(&hll_b, B.rows * (uint64_t)P));
-  mk.mark("est_malloc");
+  mk.none("est_malloc");
   OC_TRY(launch_hll_build(d.log_p, B, hll_b, s));
   mk.mark("est_hll_construct");
   const int ns = num_samples(c, A.rows);
@@ -810,13 +932,20 @@ int Run::sampling() {
                           ri.products, sprod, 1, tmp, s));
   std::vector<uint32_t> hp(ns);
   std::vector<int32_t> he(ns);
-  OC_TRY(readback(hp.data(), sprod, ns, s));
-  OC_TRY(readback(he.data(), sest, ns, s));
+  if (2ull * ns <= HostPage::kWords - HostPage::kData) {
+    const uint32_t *w;
+    OC_TRY(fetch({{sprod, (uint32_t)ns}, {sest, (uint32_t)ns}}, &w));
+    std::memcpy(hp.data(), w, (size_t)ns * 4);
+    std::memcpy(he.data(), w + ns, (size_t)ns * 4);
+  } else {
+    OC_TRY(readback(hp.data(), sprod, ns, s));
+    OC_TRY(readback(he.data(), sest, ns, s));
+  }
   mk.mark("est_sample");
   const int hl = d.hash_largest;
   decide_sampling(c, *h, hp, he, d);
   d.hash_largest = hl;
-  mk.mark("sampling_var_calc_host");
+  mk.none("sampling_var_calc_host");
   return OC_OK;
 }
 
@@ -836,7 +965,9 @@ int Run::learned_capacities(bool *use_est) {
   uint64_t *ps;
   OC_TRY(ar.get(&ps, m + 1));
   OC_TRY(launch_scan_u32(learned_est, ps, m, scan_tmp, s));
-  OC_TRY(readback(&h->learned_total, ps + m, 1, s));
+  const uint32_t *w;
+  OC_TRY(fetch({{ps + m, 2}}, &w));
+  h->learned_total = u64_at(w);
   ar.free(ps);
   h->learned_consulted = true;
   *use_est = (double)h->total_products >=
@@ -1022,7 +1153,11 @@ int Run::run_fat() {
   OC_TRY(launch_fat_count(bits, m, B.cols, nnz, s));
   fam("fat", "numeric_fat", true, nullptr, (uint32_t)m);
   mk.mark("numeric_fat");
-  OC_TRY(alloc_c_from_counts(nnz));
+  OC_TRY(c_offsets(nnz));
+  mk.mark("epilogue_scan");
+  const uint32_t *w;
+  OC_TRY(fetch({c_nnz()}, &w));
+  OC_TRY(c_entries(u64_at(w)));
   OC_TRY(launch_fat_compact(A.vtype, dense, bits, m, B.cols, (const uint64_t *)C->row_offsets,
                             C->col_ids, C->values, s));
   mk.mark("epilogue_copy");
@@ -1037,7 +1172,6 @@ int Run::run_usparse() {
   OC_TRY(ar.get(&tc, h->total_products));
   OC_TRY(ar.get(&tv, h->total_products * vsize(A.vtype)));
   OC_TRY(ar.get(&nnz, m + 1));
-  mk.mark("numeric_malloc");
   const int esc_n = std::min(d.spark_kernel_size, 64);
   NumOut o;
   std::memset(&o, 0, sizeof(o));
@@ -1048,12 +1182,11 @@ int Run::run_usparse() {
   OC_TRY(launch_esc(esc_n, acc(), o, s));
   fam("esc_all_rows", "numeric_usparse_main", true, nullptr, (uint32_t)m);
   mk.mark("numeric_usparse_main");
+  uint32_t *ovf = nullptr;
+  const uint32_t *w;
   if (h->max_products > (uint32_t)esc_n) {
-    uint32_t *ovf;
-    OC_TRY(ar.get(&ovf, m + 4));
-    o.ovf_rows = ovf + 4;
+    OC_TRY(counters(&ovf, &o.ovf_rows));
     o.ovf_count = ovf;
-    HIP_TRY(hipMemsetAsync(ovf, 0, 16, s));
     BinParams bp;
     std::memset(&bp, 0, sizeof(bp));
     bp.kind = 1;
@@ -1067,19 +1200,22 @@ int Run::run_usparse() {
     uint8_t *bor = nullptr;
     uint32_t *brows = nullptr, *boff = nullptr;
     uint32_t hoff[kBinSlots + 1];
-    OC_TRY(binning(bp, &bor, &brows, &boff, hoff));
+    OC_TRY(queue_binning(bp, &bor, &brows, &boff));
+    OC_TRY(fetch({{boff, kBinSlots + 1}}, &w));
+    std::memcpy(hoff, w, sizeof(hoff));
     std::memcpy(h->bin2, hoff, sizeof(hoff));
     h->have_bin2 = true;
     OC_TRY(numeric_bins(brows, hoff, o, true, boff));
-    uint32_t novf = 0;
-    OC_TRY(readback(&novf, ovf, 1, s));
-    if (novf) {
-      set_error("internal: %u ultra-sparse outlier rows overflowed", novf);
-      return OC_ERR_CAPACITY;
-    }
     mk.mark("numeric_usparse_outlier");
   }
-  OC_TRY(alloc_c_from_counts(nnz));
+  OC_TRY(c_offsets(nnz));
+  mk.mark("epilogue_scan");
+  OC_TRY(fetch({c_nnz(), {ovf, ovf ? 1u : 0u}}, &w));
+  if (ovf && w[2]) {
+    set_error("internal: %u ultra-sparse outlier rows overflowed", w[2]);
+    return OC_ERR_CAPACITY;
+  }
+  OC_TRY(c_entries(u64_at(w)));
   OC_TRY(launch_copy_rows(A.vtype, m, nullptr, nnz, psum_prod, nullptr, tc, tv,
                           (const uint64_t *)C->row_offsets, C->col_ids, C->values, s));
   mk.mark("epilogue_copy");
@@ -1089,11 +1225,9 @@ int Run::run_usparse() {
 int Run::run_precise() {
   const Decision &d = h->d;
   const uint64_t m = A.rows;
-  uint32_t *nnz, *ovf;
+  uint32_t *nnz, *ovf, *ovf_rows;
   OC_TRY(ar.get(&nnz, m + 1));
-  OC_TRY(ar.get(&ovf, m + 8));
-  HIP_TRY(hipMemsetAsync(ovf, 0, 32, s));
-  uint32_t *ovf_rows = ovf + 8;
+  OC_TRY(counters(&ovf, &ovf_rows));
   BinParams bp;
   std::memset(&bp, 0, sizeof(bp));
   bp.kind = 0;
@@ -1108,14 +1242,22 @@ int Run::run_precise() {
   uint8_t *bor = nullptr;
   uint32_t *brows = nullptr, *boff = nullptr;
   uint32_t hoff[kBinSlots + 1];
-  OC_TRY(binning(bp, &bor, &brows, &boff, hoff));
+  const uint32_t *w;
+  OC_TRY(queue_binning(bp, &bor, &brows, &boff));
+  OC_TRY(bitmap_offsets(bor));
+  mk.mark("symbolic_binning");
+  OC_TRY(fetch({{boff, kBinSlots + 1}, {bmoff_all ? bmoff_all + m : nullptr, bmoff_all ? 2u : 0u}},
+               &w));
+  std::memcpy(hoff, w, sizeof(hoff));
   std::memcpy(h->bin1, hoff, sizeof(hoff));
   h->have_bin1 = true;
-  mk.mark("symbolic_binning");
   const AccArgs a = acc();
   const Tables &t = tables();
-  OC_TRY(row_bitmaps(brows, hoff));
-  OC_TRY(claims());
+  if (bmoff_all) OC_TRY(row_bitmaps(u64_at(w + kBinSlots + 1)));
+  auto stage = [&](const char *name, bool work) {
+    if (work) mk.mark(name);
+    else mk.none(name);
+  };
   for (int b = 0; b <= 5; ++b) {
     const uint32_t n = hoff[b + 1] - hoff[b];
     if (!n) continue;
@@ -1125,14 +1267,14 @@ int Run::run_precise() {
                            RowSel{boff + b, nullptr, claim_ctr + b, hoff[b]}));
   }
   fam("sym_hash", "symbolic_hash", false, brows + hoff[0], hoff[6] - hoff[0]);
-  mk.mark("symbolic_hash");
+  stage("symbolic_hash", hoff[6] > hoff[0]);
   if (hoff[7] > hoff[6]) {
     OC_TRY(window_scratch());
     OC_TRY(launch_sym_window(a, brows, hoff[7] - hoff[6], h->max_a_nnz, nnz, win_scratch, s,
                              RowSel{boff + 6, nullptr, claim_ctr + 6, hoff[6]}, row_bmoff, row_bm));
   }
   fam("sym_window", "symbolic_window", false, brows + hoff[6], hoff[7] - hoff[6]);
-  mk.mark("symbolic_window");
+  stage("symbolic_window", hoff[7] > hoff[6]);
   for (int b = 7; b <= 13; ++b) {
     const uint32_t n = hoff[b + 1] - hoff[b];
     if (!n) continue;
@@ -1144,22 +1286,8 @@ int Run::run_precise() {
                             RowSel{boff + b, nullptr, claim_ctr + b, hoff[b]}));
   }
   fam("sym_dense", "symbolic_dense", false, brows + hoff[7], hoff[14] - hoff[7]);
-  mk.mark("symbolic_dense");
-  {
-    // Rows whose hash table filled up (the shrunken tables of the estimated
-    // compaction, or a symbolic expansion that undersized a bin) are
-    // recounted with the windowed bitmap, which has no size limit.
-    uint32_t n = 0;
-    OC_TRY(readback(&n, ovf, 1, s));
-    h->sym_overflow_rows = n;
-    if (n) {
-      OC_TRY(window_scratch());
-      OC_TRY(launch_sym_window(a, ovf_rows, n, h->max_a_nnz, nnz, win_scratch, s));
-    }
-    mk.mark("symbolic_overflow");
-  }
+  stage("symbolic_dense", hoff[14] > hoff[7]);
   OC_TRY(band_symbolic(nnz));
-  OC_TRY(alloc_c_from_counts(nnz));
   // numeric binning on exact counts, SpGEMM.cuh:1247-1283
   BinParams nb;
   std::memset(&nb, 0, sizeof(nb));
@@ -1174,10 +1302,31 @@ int Run::run_precise() {
   nb.skip_flag = band.flag;
   uint8_t *bor2 = nullptr;
   uint32_t *brows2 = nullptr, *boff2 = nullptr;
-  OC_TRY(binning(nb, &bor2, &brows2, &boff2, hoff));
+  // C's offsets and the numeric bins are queued as if no row had overflowed;
+  // the host reads them together with the overflow count.
+  auto counted = [&]() -> int {
+    OC_TRY(c_offsets(nnz));
+    mk.mark("epilogue_scan");
+    OC_TRY(queue_binning(nb, &bor2, &brows2, &boff2));
+    mk.mark("numeric_binning");
+    return fetch({c_nnz(), {boff2, kBinSlots + 1}, {ovf, 1}}, &w);
+  };
+  OC_TRY(counted());
+  h->sym_overflow_rows = w[2 + kBinSlots + 1];
+  mk.none("symbolic_overflow");
+  if (h->sym_overflow_rows) {
+    // Rows whose hash table filled up (the shrunken tables of the estimated
+    // compaction, or a symbolic expansion that undersized a bin) are
+    // recounted with the windowed bitmap, which has no size limit.
+    OC_TRY(window_scratch());
+    OC_TRY(launch_sym_window(a, ovf_rows, h->sym_overflow_rows, h->max_a_nnz, nnz, win_scratch, s));
+    mk.mark("symbolic_overflow");
+    OC_TRY(counted());
+  }
+  std::memcpy(hoff, w + 2, sizeof(hoff));
   std::memcpy(h->bin2, hoff, sizeof(hoff));
   h->have_bin2 = true;
-  mk.mark("numeric_binning");
+  OC_TRY(c_entries(u64_at(w)));
   NumOut o;
   std::memset(&o, 0, sizeof(o));
   o.off = (const uint64_t *)C->row_offsets;
@@ -1188,11 +1337,12 @@ int Run::run_precise() {
   o.nnz_hint = nnz;
   OC_TRY(numeric_bins(brows2, hoff, o, true, boff2));
   OC_TRY(band_numeric(o));
-  // exact capacities cannot overflow; recount defensively if one did
-  uint32_t n = 0;
-  OC_TRY(readback(&n, ovf + 1, 1, s));
-  h->precise_recount = n;
-  OC_TRY(big_rows(ovf_rows, n, o));
+  // exact capacities cannot overflow; recounted defensively if one did, once
+  // the stream has drained (finish_precise)
+  OC_TRY(publish({{ovf + 1, 1}}));
+  recount.pending = true;
+  recount.rows = ovf_rows;
+  recount.o = o;
   if (h->keep_plan) {
     // a whole-path replay needs the window scratch and the tile tables
     // even when this run had no rows for them
@@ -1246,21 +1396,33 @@ int Run::run_precise() {
     p.band_ts = band.ts;
     p.band_counter = band.counter;
     p.band_pref = band.pref;
-    p.valid = n == 0;  // a recount would make the numeric phase two-step
+    p.valid = true;  // finish_precise clears it after a recount
   }
+  return OC_OK;
+}
+
+// After the precise workflow's stream has drained: recomputes the rows that
+// its numeric kernels listed (there are none unless a count was wrong).
+int Run::finish_precise() {
+  const uint32_t *w;
+  OC_TRY(await(&w));
+  const uint32_t n = h->precise_recount = *w;
+  recount.pending = false;
+  if (!n) return OC_OK;
+  if (h->keep_plan) h->plan.valid = false;  // a replay would need the second step
+  OC_TRY(big_rows(recount.rows, n, recount.o));
+  HIP_TRY(hipStreamSynchronize(s));
   return OC_OK;
 }
 
 int Run::run_est() {
   const Decision &d = h->d;
   const uint64_t m = A.rows;
-  uint32_t *est, *nnz, *ovf;
+  uint32_t *est, *nnz, *ovf, *ovf_rows;
   OC_TRY(ar.get(&est, m + 1));
   OC_TRY(ar.get(&nnz, m + 1));
-  OC_TRY(ar.get(&ovf, m + 8));
-  HIP_TRY(hipMemsetAsync(ovf, 0, 32, s));
-  uint32_t *ovf_rows = ovf + 8;
-  mk.mark("est_malloc");
+  OC_TRY(counters(&ovf, &ovf_rows));
+  mk.none("est_malloc");
   if (h->est_override) {
     HIP_TRY(hipMemcpyAsync(est, h->est_override, m * 4, hipMemcpyDeviceToDevice, s));
   } else if (h->learned_run) {
@@ -1292,14 +1454,17 @@ int Run::run_est() {
   uint8_t *bor = nullptr;
   uint32_t *brows = nullptr, *boff = nullptr;
   uint32_t hoff[kBinSlots + 1];
-  OC_TRY(binning(bp, &bor, &brows, &boff, hoff));
-  std::memcpy(h->bin2, hoff, sizeof(hoff));
-  h->have_bin2 = true;
+  const uint32_t *w;
+  OC_TRY(queue_binning(bp, &bor, &brows, &boff));
   uint64_t *psum_est;
   OC_TRY(ar.get(&psum_est, m + 1));
   OC_TRY(launch_scan_u32(est, psum_est, m, scan_tmp, s));
-  OC_TRY(readback(&h->total_est, psum_est + m, 1, s));
   mk.mark("numeric_binning");
+  OC_TRY(fetch({{boff, kBinSlots + 1}, {psum_est + m, 2}}, &w));
+  std::memcpy(hoff, w, sizeof(hoff));
+  std::memcpy(h->bin2, hoff, sizeof(hoff));
+  h->have_bin2 = true;
+  h->total_est = u64_at(w + kBinSlots + 1);
   // estimated slots plus a spare region for the rows that outgrow theirs
   // (SpGEMM.cuh:1560-1587)
   const double coe = c.hll_numeric_malloc_expansion_coe;
@@ -1308,10 +1473,8 @@ int Run::run_est() {
     // The estimated region and C are held at once (C is at least the
     // estimate's size).  When both would take more than 60% of the device,
     // the precise workflow, which holds only C, runs instead.
-    size_t fr = 0, tot = 0;
-    HIP_TRY(hipMemGetInfo(&fr, &tot));
     const double bytes = (double)(cap_total + h->total_est) * (double)(4 + vsize(A.vtype));
-    if (bytes > 0.6 * (double)tot) {
+    if (bytes > 0.6 * (double)h->dev_bytes) {
       h->est_memory_fallback = true;
       h->d.ana2_type = 0;
       h->learned_run = false;
@@ -1345,28 +1508,36 @@ int Run::run_est() {
     fam("num_window", "numeric_window", true, brows + hoff[13], n13);
     mk.mark("numeric_window");
   }
-  uint32_t n1 = 0;
-  OC_TRY(readback(&n1, ovf, 1, s));
+  // C's offsets are queued as if no row had outgrown its slot; the host
+  // reads C's size together with the overflow count
+  auto counted = [&]() -> int {
+    OC_TRY(c_offsets(nnz));
+    mk.mark("epilogue_scan");
+    return fetch({c_nnz(), {ovf, 1}}, &w);
+  };
+  OC_TRY(counted());
+  const uint32_t n1 = w[2];
   const uint32_t nmove = inplace13 ? 0u : n13;
   if (nmove)
     HIP_TRY(hipMemcpyAsync(ovf_rows + n1, brows + hoff[13], (size_t)nmove * 4,
                            hipMemcpyDeviceToDevice, s));
   const uint32_t novf = n1 + nmove;
   h->overflow_rows = n1;
-  uint64_t *src_off;
-  OC_TRY(ar.get(&src_off, m + 1));
-  HIP_TRY(hipMemcpyAsync(src_off, psum_est, (m + 1) * 8, hipMemcpyDeviceToDevice, s));
+  uint64_t *src_off = psum_est;
   bool separate = false;  // overflow rows in a buffer of their own
   uint32_t *sc = nullptr;
   uint8_t *sv = nullptr;
+  mk.none("numeric_overflow");
   if (novf) {
+    OC_TRY(ar.get(&src_off, m + 1));
+    HIP_TRY(hipMemcpyAsync(src_off, psum_est, (m + 1) * 8, hipMemcpyDeviceToDevice, s));
     unsigned long long *used;
     OC_TRY(ar.get(&used, 1));
     HIP_TRY(hipMemsetAsync(used, 0, 8, s));
     OC_TRY(launch_assign_spare(ovf_rows, novf, ri.products, ri.left, ri.right,
                                h->total_est, used, src_off, s));
-    unsigned long long hu = 0;
-    OC_TRY(readback(&hu, used, 1, s));
+    OC_TRY(fetch({{used, 2}}, &w));
+    const uint64_t hu = u64_at(w);
     h->est_spare_need = hu;
     NumOut o2 = o;
     o2.cap = nullptr;
@@ -1386,11 +1557,12 @@ int Run::run_est() {
       o2.vals = sv;
     }
     OC_TRY(big_rows(ovf_rows, novf, o2));
+    mk.mark("numeric_overflow");
+    OC_TRY(counted());
   }
   h->est_separate_spare = separate;
   fam("num_overflow", "numeric_overflow", true, ovf_rows, novf);
-  mk.mark("numeric_overflow");
-  OC_TRY(alloc_c_from_counts(nnz));
+  OC_TRY(c_entries(u64_at(w)));
   if (!separate) {
     OC_TRY(launch_copy_rows(A.vtype, m, nullptr, nnz, src_off, nullptr, tc, tv,
                             (const uint64_t *)C->row_offsets, C->col_ids, C->values, s));
@@ -1734,6 +1906,10 @@ int spgemm_impl(oc_spgemm *h, const oc_csr *dA, const oc_csr *dB, oc_csr *dC,
                dA->col_ids, dA->values, dA->vtype};
   r.B = DevCsr{dB->rows, dB->cols, dB->nnz, (const uint32_t *)dB->row_offsets,
                dB->col_ids, dB->values, dB->vtype};
+  if (!h->dev_bytes) {
+    size_t fr = 0;
+    HIP_TRY(hipMemGetInfo(&fr, &h->dev_bytes));
+  }
   r.mk.mark("start");
   int rc = OC_OK;
   if (dA->rows == 0) {
@@ -1816,6 +1992,7 @@ int spgemm_impl(oc_spgemm *h, const oc_csr *dA, const oc_csr *dB, oc_csr *dC,
     set_error("stream error: %s", hipGetErrorString(e));
     rc = OC_ERR_HIP;
   }
+  if (rc == OC_OK && r.recount.pending) rc = r.finish_precise();
   r.mk.resolve(h->stage_ms, h->total_ms);
   if (rc == OC_OK && h->keep_plan && h->plan.valid) {
     // the plan keeps this run's memory for replays (freed by drop_plan);
@@ -1825,9 +2002,7 @@ int spgemm_impl(oc_spgemm *h, const oc_csr *dA, const oc_csr *dB, oc_csr *dC,
     r.ar.recs.clear();
   } else {
     if (h->keep_plan) h->plan.valid = false;
-    size_t fr = 0, tot = 0;
-    if (e == hipSuccess && hipMemGetInfo(&fr, &tot) == hipSuccess && h->mem.total() > tot / 4)
-      h->mem.trim();
+    if (e == hipSuccess && h->mem.total() > h->dev_bytes / 4) h->mem.trim();
     (void)hipGetLastError();
     r.ar.recs.clear();
   }
@@ -1953,7 +2128,7 @@ int full_replay_impl(oc_spgemm *h, hipStream_t s) {
   }
   // symbolic: binning, then every bin persistent over its device range
   OC_TRY(launch_binning(p.sym_bp, m, p.bor1, p.brows1, p.boff1, p.bin_tmp, s));
-  uint32_t *ovf_rows = p.ovf + 8;
+  uint32_t *ovf_rows = p.ovf + Run::kCtlWords;
   for (int b = 0; b <= 5; ++b) {
     const uint32_t S = t.hash_sym[b];
     OC_TRY(launch_sym_hash(b, a, p.brows1, 0, p.est_symbolic ? S - S / 8 : S, p.nnz, ovf_rows,
