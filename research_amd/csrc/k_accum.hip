@@ -368,16 +368,20 @@ __device__ __forceinline__ uint32_t list_heavy(const KA &a, const RowHead &rh, u
   return n <= cap ? n : 0u;
 }
 
-// Persistent row loop over the rows [bounds[0], bounds[1]) of a bin list:
-// chunks of kClaimRows rows claimed from *claim (zeroed before the launches).
-// A workgroup that starts late or draws costly rows takes fewer chunks;
-// each workgroup striding over a fixed share of the rows ran the bins
-// 10-40% slower than launching one workgroup per row.  One loop latch,
-// after the barriers that publish the claim.
+// The rows of a bin kernel:
+//  - the workgroup's own (no bounds: one workgroup per row);
+//  - without a claim counter, the rows [bounds[0], bounds[1]) by a stride of
+//    the grid (which is then about as many workgroups as rows);
+//  - else those rows in chunks claimed from *claim (zeroed before the
+//    launches).  A workgroup that starts late or draws costly rows takes
+//    fewer chunks; striding with a grid of only the resident workgroups ran
+//    the bins 10-40% slower than launching one workgroup per row.
+// One call of `row` for all three, so its code is there once, and one latch
+// of the claim loop, after the barriers that publish the claim.
 constexpr uint32_t kClaimRows = 16;
 template <typename F>
-__device__ __forceinline__ void claim_rows(const uint32_t *__restrict__ bounds, uint32_t *claim,
-                                           F &&row) {
+__device__ __forceinline__ void bin_rows(const uint32_t *__restrict__ bounds, uint32_t *claim,
+                                         F &&row) {
   // The claim is published in the first word of the dynamic LDS, which no
   // row keeps between rows (each row initialises its LDS).  A static slot
   // would add LDS to every launch of the kernel: 4 bytes moved the dynamic
@@ -391,39 +395,32 @@ __device__ __forceinline__ void claim_rows(const uint32_t *__restrict__ bounds, 
   // degree 32: windowed symbolic rows 33.1 -> 9.6 ms; the 48 panels of
   // that product 3.09 -> 2.17 s).
   extern __shared__ uint32_t s_claim[];
-  const uint32_t b0 = bounds[0], b1 = bounds[1];
-  const uint32_t n = b1 - min(b0, b1);
-  const uint32_t chunk = max(1u, min(kClaimRows, n / (16u * gridDim.x)));
-  for (;;) {
-    if (threadIdx.x == 0) s_claim[0] = atomicAdd(claim, chunk);
-    __syncthreads();
-    const uint32_t c = s_claim[0];
-    __syncthreads();
-    if (c >= n) break;
-    const uint32_t e = min(b1, b0 + c + chunk);
-    for (uint32_t i = b0 + c; i < e; ++i) {
-      row(i);
-      __syncthreads();  // the next row re-initialises the LDS
-    }
+  uint64_t i = blockIdx.x, e = i + 1;
+  uint32_t b0 = 0, b1 = 0, n = 0, chunk = 0, step = 1;
+  if (bounds) {
+    b0 = bounds[0];
+    b1 = bounds[1];
+    n = b1 - min(b0, b1);
+    chunk = max(1u, min(kClaimRows, n / (16u * gridDim.x)));
+    i += b0;
+    e = b1;
+    step = claim ? 1u : gridDim.x;
   }
-}
-
-// The rows of a bin kernel: the workgroup's own (one workgroup per row), the
-// rows [bounds[0], bounds[1]) by claims, or, without a claim counter, by a
-// stride of the grid (which is then about as many workgroups as rows).
-template <typename F>
-__device__ __forceinline__ void bin_rows(const uint32_t *__restrict__ bounds, uint32_t *claim,
-                                         F &&row) {
-  if (!bounds) {
-    row(blockIdx.x);
-  } else if (claim) {
-    claim_rows(bounds, claim, row);
-  } else {
-    const uint32_t b0 = bounds[0], b1 = bounds[1];
-    for (uint64_t i = (uint64_t)b0 + blockIdx.x; i < b1; i += gridDim.x) {
+  for (;;) {
+    if (claim) {
+      if (threadIdx.x == 0) s_claim[0] = atomicAdd(claim, chunk);
+      __syncthreads();
+      const uint32_t c = s_claim[0];
+      __syncthreads();
+      if (c >= n) break;
+      i = (uint64_t)b0 + c;
+      e = min((uint64_t)b1, i + chunk);
+    }
+    for (; i < e; i += step) {
       row((uint32_t)i);
       __syncthreads();  // the next row re-initialises the LDS
     }
+    if (!claim) break;
   }
 }
 
@@ -438,6 +435,47 @@ __device__ __forceinline__ void bin_rows(const uint32_t *__restrict__ bounds, ui
 // caller sweeps them).  f(c, v, ok) takes U columns, B values times the A
 // value (VALS) and whether the lane has a product there, and returns false
 // (the whole wave) to stop.  All lanes of the workgroup call it.
+//
+// flat_owner: the B entry (q) and A value (pa) of product p0 + lane of a
+// chunk, whose lane j holds the length, start (ex), B position less the start
+// (base) and A value of its j-th B row; false past the chunk's P products.
+// The B row of a product is the last non-empty one that starts at or before
+// it.
+template <bool VALS, typename T>
+__device__ __forceinline__ bool flat_owner(uint32_t p0, uint32_t P, uint32_t len, uint32_t ex,
+                                           uint32_t base, T av, uint32_t &q, T &pa) {
+  const uint32_t p = p0 + (uint32_t)lane_id();
+  const uint64_t here = __ballot(len != 0 && ex <= p0);
+  uint64_t starts = __ballot(len != 0 && ex > p0 && ex - p0 < kWave);
+  const int first = 63 - __clzll(here);
+  if (starts == 0) {  // one B row gives the whole block
+    q = (uint32_t)__builtin_amdgcn_readlane((int)base, first) + p;
+    if (VALS) pa = __shfl(av, first);
+    return p < P;
+  }
+  int owner = first;
+  if (__popcll(starts) <= 12) {
+    do {
+      const int t = __builtin_ctzll(starts);
+      starts &= starts - 1;
+      const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)ex, t);
+      owner = p >= e ? t : owner;
+    } while (starts);
+  } else {
+    // many short B rows: a binary search of the ascending starts (an empty
+    // row's start is that of the row after it)
+    owner = 0;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      const uint32_t e = __shfl(ex, owner + d);
+      owner = e <= p ? owner + d : owner;
+    }
+  }
+  q = __shfl(base, owner) + p;
+  if (VALS) pa = __shfl(av, owner);
+  return p < P;
+}
+
 template <int BS, int U, bool VALS, typename T, typename F>
 __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uint32_t a1,
                                              uint32_t share, uint32_t skip, F &&f) {
@@ -484,40 +522,8 @@ __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uin
         q[u] = 0;
         pa[u] = T(0);
         ok[u] = false;
-        if (b + u < b1) {  // uniform
-          // the A entry of product p: the last non-empty one that starts at
-          // or before it
-          const uint32_t p0 = (b + u) * kWave, p = p0 + lane;
-          ok[u] = p < P;
-          const uint64_t here = __ballot(len != 0 && ex <= p0);
-          uint64_t starts = __ballot(len != 0 && ex > p0 && ex - p0 < kWave);
-          const int first = 63 - __clzll(here);
-          if (starts == 0) {  // one B row gives the whole block
-            q[u] = (uint32_t)__builtin_amdgcn_readlane((int)base, first) + p;
-            if (VALS) pa[u] = __shfl(av, first);
-          } else {
-            int owner = first;
-            if (__popcll(starts) <= 12) {
-              do {
-                const int t = __builtin_ctzll(starts);
-                starts &= starts - 1;
-                const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)ex, t);
-                owner = p >= e ? t : owner;
-              } while (starts);
-            } else {
-              // many short B rows: the last of the ascending starts at or
-              // before p (an empty row's start is that of the row after it)
-              owner = 0;
-#pragma unroll
-              for (int d = 32; d > 0; d >>= 1) {
-                const uint32_t e = __shfl(ex, owner + d);
-                owner = e <= p ? owner + d : owner;
-              }
-            }
-            q[u] = __shfl(base, owner) + p;
-            if (VALS) pa[u] = __shfl(av, owner);
-          }
-        }
+        if (b + u < b1)  // uniform
+          ok[u] = flat_owner<VALS>((b + u) * kWave, P, len, ex, base, av, q[u], pa[u]);
       }
       uint32_t c[U];
       T v[U];
@@ -550,6 +556,9 @@ __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uin
 // rows of 576 products in B rows of 24, 717 -> 534 us; numeric hash rows of
 // the same product 730 -> 684 us; 131,072 banded rows of 33 x 33, numeric
 // dense, 325 -> 221 us.)
+// (Numeric hash rows of one chunk go product by product too: their few B
+// rows, however long, are then shared evenly by all waves.  R-MAT 2^18, 1024
+// threads: 1431 -> 1291 us.)
 constexpr uint32_t kFlatAvg = 64;
 
 // Waves per chunk of for_products: enough blocks of 64 products for each (U
@@ -560,7 +569,7 @@ __device__ __forceinline__ uint32_t flat_share(uint32_t nA, uint32_t avg) {
   if constexpr (NW == 1) return 1u;
   const uint32_t chunks = (nA + kWave - 1) / kWave;
   uint32_t share = 1;
-  while (share < NW && (2 * share * U <= avg || NW / share > chunks)) share *= 2;
+  while (share < NW && (2 * share * U <= avg || NW / share > chunks)) share *= 2;  // 2^k
   return share;
 }
 
@@ -887,6 +896,231 @@ __host__ __device__ inline HashLayout hash_layout(uint32_t S, uint32_t nwaves) {
   return L;
 }
 
+// f(t, ck[t]) over one bucket's keys: eight reads in flight in a long one
+// (the largest buckets of an R-MAT row hold a few percent of its keys, and
+// one read at a time took 20,000 cycles of a 1024-thread row).
+template <typename F>
+__device__ __forceinline__ void for_bucket(const uint32_t *ck, uint32_t s0, uint32_t s1, F &&f) {
+  uint32_t t = s0;
+  for (; t + 8 <= s1; t += 8) {
+    uint32_t k[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) k[u] = ck[t + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) f(t + u, k[u]);
+  }
+  for (; t < s1; ++t) f(t, ck[t]);
+}
+
+// Numeric rows without a hash table: the row's products are sorted by column
+// directly.  A row of at most 64 A entries whose products fit the LDS keeps
+// them in registers (U per lane, all gathers in flight at once), counts them
+// into buckets by the top bits of their column, places them by bucket, and
+// compares each with the few others of its bucket: the smaller ones give its
+// place, the equal ones are duplicates, which the first of them sums.  That
+// is about 11 LDS operations for 64 products.  A hash table costs its
+// clearing, a compare-and-swap with its collisions and two sweeps over the
+// table to order the output (44 for the rows below), and pays only where
+// many products meet in one output, which these rows, bounded by their
+// products, do not have room for.  Returns false, having written nothing,
+// for a row it does not take: the table's path follows.  (85,720 Erdos-Renyi
+// rows of 576 products: 684 -> @SR1@ us; R-MAT 2^18's rows of the largest
+// tables: 1411 -> @SR2@ us.)
+//
+// LDS: header, bucket starts and duplicate counts (u16, 4 BS each), then the
+// products' columns and values in bucket order.
+template <int BS>
+struct SortRows {
+  static constexpr int U = 5;                      // products per lane at most
+  static constexpr int kLogBuckets = __builtin_ctz(BS) + 2;
+  static constexpr uint32_t kCrowded = 192;        // most products of one bucket
+  static constexpr uint32_t off_start = 1280, off_dup = off_start + 8 * BS + 8,
+                            off_val = off_dup + 8 * BS + 8;
+  __host__ __device__ static uint32_t capacity(uint32_t bytes) {
+    return bytes > off_val ? (bytes - off_val) / 12 : 0u;
+  }
+};
+
+template <int BS, typename T, bool EST>
+__device__ __forceinline__ bool num_sort_row(const KArgs<T> &a, uint32_t r, const RowHead &rh,
+                                             uint64_t off, uint32_t cap, uint32_t lds_bytes,
+                                             const KOut<T> &o) {
+  using SR = SortRows<BS>;
+  constexpr uint32_t NW = BS / kWave;
+  constexpr int U = SR::U;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const uint32_t nA = rh.a1 - rh.a0, P = rh.prod;
+  const uint32_t nb = (P + kWave - 1) / kWave, per = (nb + NW - 1) / NW;
+  if (BS > 512 || nA == 0 || nA > kWave || P == 0 || per > (uint32_t)U || P > SR::capacity(lds_bytes) ||
+      rh.right - rh.left >= 0x80000000u)
+    return false;
+  uint32_t *hdr = reinterpret_cast<uint32_t *>(smem);
+  uint32_t *dsum = reinterpret_cast<uint32_t *>(smem + 256);
+  uint32_t *bw = reinterpret_cast<uint32_t *>(smem + SR::off_start);  // two buckets a word
+  uint16_t *start = reinterpret_cast<uint16_t *>(bw);
+  uint32_t *dw = reinterpret_cast<uint32_t *>(smem + SR::off_dup);
+  const uint16_t *dup = reinterpret_cast<const uint16_t *>(dw);
+  double *cv = reinterpret_cast<double *>(smem + SR::off_val);
+  uint32_t *ck = reinterpret_cast<uint32_t *>(cv + SR::capacity(lds_bytes));
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wid =
+      NW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t lo = rh.left;
+  const int span_bits = rh.right > lo ? 32 - __clz(rh.right - lo) : 0;
+  const uint32_t sh = (uint32_t)max(0, span_bits - SR::kLogBuckets);
+  reinterpret_cast<uint2 *>(bw)[threadIdx.x] = make_uint2(0u, 0u);
+  reinterpret_cast<uint2 *>(dw)[threadIdx.x] = make_uint2(0u, 0u);
+  if (threadIdx.x == 0) {
+    hdr[4] = hdr[5] = 0;
+    start[4 * BS] = (uint16_t)P;
+  }
+  // this wave's products (blocks of 64, as in for_products with one chunk)
+  uint32_t key[U];
+  double pv[U];
+  const uint32_t b0 = min(nb, wid * per), b1 = min(nb, b0 + per);
+  const uint32_t pend = min(P, b1 * kWave), pme = b0 * kWave + lane;
+  auto ok = [&](int u) { return pme + u * kWave < pend; };
+  {
+    uint32_t bs = 0, be = 0;
+    T av = T(0);
+    if (lane < nA) {
+      const uint32_t k = a.a_ci[rh.a0 + lane];
+      av = a.a_v[rh.a0 + lane];
+      bs = a.b_rp[k];
+      be = a.b_rp[k + 1];
+    }
+    auto add = [](uint32_t x, uint32_t y) { return x + y; };
+    const uint32_t len = be - bs, incl = wave_incl_scan(len, 0u, add);
+    const uint32_t ex = incl - len, base = bs - ex;
+    T pa[U], v[U];
+    uint32_t q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      q[u] = 0;
+      pa[u] = T(0);
+      if (b0 + u < b1) flat_owner<true>((b0 + u) * kWave, P, len, ex, base, av, q[u], pa[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      key[u] = lo;
+      v[u] = T(0);
+      if (ok(u)) {
+        key[u] = a.b_ci[q[u]];
+        v[u] = a.b_v[q[u]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      pv[u] = product_pz((double)pa[u], (double)v[u]);
+      key[u] -= lo;
+    }
+  }
+  __syncthreads();
+  uint32_t arr[U];  // arrival number in the bucket
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    arr[u] = 0;
+    if (ok(u)) {
+      const uint32_t b = key[u] >> sh, half = 16 * (b & 1);
+      arr[u] = (atomicAdd(&bw[b >> 1], 1u << half) >> half) & 0xFFFFu;
+    }
+  }
+  __syncthreads();
+  uint2 *mine4 = reinterpret_cast<uint2 *>(bw) + threadIdx.x;  // a thread's four buckets
+  const uint2 cw = *mine4;
+  const uint32_t n0 = cw.x & 0xFFFFu, n1 = cw.x >> 16, n2 = cw.y & 0xFFFFu, n3 = cw.y >> 16;
+  if (max(max(n0, n1), max(n2, n3)) > SR::kCrowded) hdr[4] = 1;
+  uint32_t tot;
+  const uint32_t st = block_excl_sum(n0 + n1 + n2 + n3, dsum, &tot);
+  *mine4 = make_uint2(st | (st + n0) << 16, (st + n0 + n1) | (st + n0 + n1 + n2) << 16);
+  __syncthreads();
+  if (hdr[4]) {
+    __syncthreads();  // every wave has read the flag
+    return false;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (ok(u)) {
+      const uint32_t pos = start[key[u] >> sh] + arr[u];
+      ck[pos] = key[u];
+      cv[pos] = pv[u];
+    }
+  __syncthreads();
+  // item i = threadIdx.x + u BS: the smaller keys of its bucket; a key that
+  // an earlier item of the bucket has too is a duplicate (top bit)
+  constexpr uint32_t kDup = 0x80000000u;
+  uint32_t less[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t i = threadIdx.x + u * BS;
+    less[u] = kDup;
+    if (i < P) {
+      const uint32_t kk = ck[i] & ~kDup, b = kk >> sh;
+      const uint32_t s0 = start[b], s1 = start[b + 1];
+      uint32_t n = 0;
+      bool first = true;
+      for (uint32_t t = s0; t < s1; ++t) {
+        const uint32_t kt = ck[t] & ~kDup;
+        n += kt < kk ? 1u : 0u;
+        if (kt == kk && t < i) first = false;
+      }
+      less[u] = s0 + n;
+      if (!first) {
+        less[u] = kDup;
+        ck[i] = kk | kDup;
+        atomicAdd(&dw[b >> 1], 1u << (16 * (b & 1)));
+        hdr[5] = 1;
+      }
+    }
+  }
+  __syncthreads();
+  uint32_t n = P;
+  const bool dups = hdr[5] != 0;
+  if (dups) {  // duplicates of the buckets before each bucket
+    uint2 *d4 = reinterpret_cast<uint2 *>(dw) + threadIdx.x;
+    const uint2 dv = *d4;
+    const uint32_t m0 = dv.x & 0xFFFFu, m1 = dv.x >> 16, m2 = dv.y & 0xFFFFu, m3 = dv.y >> 16;
+    uint32_t nd;
+    const uint32_t ds = block_excl_sum(m0 + m1 + m2 + m3, dsum, &nd);
+    *d4 = make_uint2(ds | (ds + m0) << 16, (ds + m0 + m1) | (ds + m0 + m1 + m2) << 16);
+    if (threadIdx.x == 0) dw[2 * BS] = nd;  // dup[4 BS]
+    n = P - nd;
+    __syncthreads();
+  }
+  if (EST && n > cap) {
+    if (threadIdx.x == 0) o.ovf_rows[atomicAdd(o.ovf_count, 1u)] = r;
+    return true;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t i = threadIdx.x + u * BS;
+    if (i >= P || less[u] == kDup) continue;
+    const uint32_t kk = ck[i];
+    double sum = cv[i];
+    uint32_t pos = less[u];
+    if (dups) {
+      const uint32_t b = kk >> sh, d0 = dup[b];
+      pos -= d0;
+      if (dup[b + 1] != d0) {
+        // duplicates in this bucket: those of smaller keys give their places
+        // up, those of this key are added
+        const uint32_t s1 = start[b + 1];
+        for (uint32_t t = start[b]; t < s1; ++t) {
+          const uint32_t kt = ck[t];
+          if (!(kt & kDup)) continue;
+          const uint32_t kv = kt & ~kDup;
+          pos -= kv < kk ? 1u : 0u;
+          if (kv == kk) sum += cv[t];
+        }
+      }
+    }
+    o.cols[off + pos] = lo + kk;
+    o.vals[off + pos] = (T)sum;
+  }
+  if (o.nnz && threadIdx.x == 0) o.nnz[r] = n;
+  return true;
+}
+
 template <int BS, typename T, bool EST>
 __device__ __forceinline__ void num_hash_row(KArgs<T> a,
                                                  uint32_t r,
@@ -904,6 +1138,7 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
   const RowHead rh = row_head(a, r);
   const uint64_t off = o.off[r];
   const uint32_t cap = EST ? o.cap[r] : 0u;
+  if (num_sort_row<BS, T, EST>(a, r, rh, off, cap, L.bytes, o)) return;
   for (uint32_t i = threadIdx.x; i < S; i += BS) {
     keys[i] = kEmpty;
     vals[i] = 0.0;
@@ -962,7 +1197,7 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
   };
   uint32_t nheavy;  // heavy B rows listed and swept by the whole workgroup
   const uint32_t avg = a1 > a0 ? rh.prod / (a1 - a0) : 0u;
-  if (avg < kFlatAvg) {
+  if (avg < kFlatAvg || a1 - a0 <= kWave) {
     const Flat fl = flat_plan<BS, 4>(a, rh, avg, &hdr[3], hdr + 8, kSymHeavy);
     nheavy = fl.listed;
     for_products<BS, 4, true>(
@@ -1108,7 +1343,7 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
         const uint32_t kk = ck[i], b = (kk - lo) >> sh;
         const uint32_t s0 = b ? bend[b - 1] : 0u, s1 = bend[b];
         uint32_t pos = s0;
-        for (uint32_t t = s0; t < s1; ++t) pos += ck[t] < kk ? 1u : 0u;
+        for_bucket(ck, s0, s1, [&](uint32_t, uint32_t kt) { pos += kt < kk ? 1u : 0u; });
         o.cols[off + pos] = kk;
         o.vals[off + pos] = (T)vals[ci[i]];
       }
@@ -1152,6 +1387,7 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
   if (o.nnz && threadIdx.x == 0) o.nnz[r] = n;
 }
 
+// (eight waves per SIMD: the bins fill the CU's waves)
 template <int BS, typename T, bool EST>
 __global__ __launch_bounds__(BS) void k_num_hash(KArgs<T> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, const uint32_t *__restrict__ err, HashLayout L, KOut<T> o, int key_bits,
