@@ -653,7 +653,26 @@ int launch_murmur(const uint32_t *cols, uint32_t *out, uint64_t n, hipStream_t s
 
 // ------------------------------------------------------------------- HLL
 // Sketch of each B row: 16 lanes per row, registers in LDS, merged with
-// LDS atomicMax (kernels/HLL.cuh:12-24, 29-103).
+// LDS atomicMax (kernels/HLL.cuh:12-24, 29-103).  A row of more than
+// kHllLong entries is left to the whole workgroup, which sweeps its listed
+// rows together: one hub on 16 lanes was the kernel's time (R-MAT 2^20, its
+// longest row 39,618 entries: 670 -> 196 us; 2^18: 260 -> 58 us).
+constexpr uint32_t kHllLong = 512;
+
+// f(column) over entries j, j + step, ... < e, four loads in flight
+template <typename F>
+__device__ __forceinline__ void hll_entries(const uint32_t *__restrict__ ci, uint32_t j,
+                                            uint32_t e, uint32_t step, F &&f) {
+  for (; j < e && e - j > 3 * step; j += 4 * step) {
+    const uint32_t c0 = ci[j], c1 = ci[j + step], c2 = ci[j + 2 * step], c3 = ci[j + 3 * step];
+    f(c0);
+    f(c1);
+    f(c2);
+    f(c3);
+  }
+  for (; j < e; j += step) f(ci[j]);
+}
+
 template <int LOGP>
 __global__ __launch_bounds__(256) void k_hll_build(const uint32_t *__restrict__ rp,
                                                    const uint32_t *__restrict__ ci,
@@ -662,25 +681,50 @@ __global__ __launch_bounds__(256) void k_hll_build(const uint32_t *__restrict__ 
   constexpr int P = 1 << LOGP;
   constexpr uint32_t CAP = 33 - LOGP;
   __shared__ uint32_t regs[16][P];
+  __shared__ uint32_t long_rows[16], nlong;
   const int g = threadIdx.x / 16, lig = threadIdx.x % 16;
-  for (uint32_t r = blockIdx.x * 16 + g; r < rows; r += gridDim.x * 16) {
-    for (int i = lig; i < P; i += 16) regs[g][i] = 0;
-    wave_sync();
-    for (uint32_t j = rp[r] + lig; j < rp[r + 1]; j += 16) {
-      const uint32_t h = murmur3_col(ci[j]);
-      const uint32_t item = min((uint32_t)__clz(h) + 1u, CAP);
-      atomicMax(&regs[g][h & (P - 1)], item);
-    }
-    wave_sync();
-    constexpr int BPL = P / 16;  // bytes per lane
+  auto into = [](uint32_t *reg, uint32_t col) {
+    const uint32_t h = murmur3_col(col);
+    atomicMax(&reg[h & (P - 1)], min((uint32_t)__clz(h) + 1u, CAP));
+  };
+  constexpr int BPL = P / 16;  // bytes per lane
+  auto store = [&](const uint32_t *reg, uint32_t r, int l) {
     uint32_t packed = 0;
 #pragma unroll
-    for (int i = 0; i < BPL; ++i) packed |= regs[g][lig * BPL + i] << (8 * i);
+    for (int i = 0; i < BPL; ++i) packed |= reg[l * BPL + i] << (8 * i);
     if (BPL == 4)
-      reinterpret_cast<uint32_t *>(out + (uint64_t)r * P)[lig] = packed;
+      reinterpret_cast<uint32_t *>(out + (uint64_t)r * P)[l] = packed;
     else
-      reinterpret_cast<uint16_t *>(out + (uint64_t)r * P)[lig] = (uint16_t)packed;
-    wave_sync();
+      reinterpret_cast<uint16_t *>(out + (uint64_t)r * P)[l] = (uint16_t)packed;
+  };
+  for (uint64_t r0 = (uint64_t)blockIdx.x * 16; r0 < rows; r0 += (uint64_t)gridDim.x * 16) {
+    if (threadIdx.x == 0) nlong = 0;
+    __syncthreads();
+    const uint64_t r = r0 + g;
+    if (r < rows) {
+      const uint32_t s = rp[r], e = rp[r + 1];
+      if (e - s > kHllLong) {
+        if (lig == 0) long_rows[atomicAdd(&nlong, 1u)] = (uint32_t)r;
+      } else {
+        for (int i = lig; i < P; i += 16) regs[g][i] = 0;
+        wave_sync();
+        hll_entries(ci, s + lig, e, 16, [&](uint32_t c) { into(regs[g], c); });
+        wave_sync();
+        store(regs[g], (uint32_t)r, lig);
+      }
+    }
+    __syncthreads();
+    const uint32_t n = nlong;
+    for (uint32_t k = 0; k < n; ++k) {  // each with a register set of its own
+      for (int i = threadIdx.x; i < P; i += 256) regs[k][i] = 0;
+      __syncthreads();
+      const uint32_t lr = long_rows[k];
+      hll_entries(ci, rp[lr] + threadIdx.x, rp[lr + 1], 256,
+                  [&](uint32_t c) { into(regs[k], c); });
+    }
+    __syncthreads();
+    if (g < (int)n) store(regs[g], long_rows[g], lig);
+    __syncthreads();  // the next rows clear the registers
   }
 }
 
@@ -701,13 +745,14 @@ int launch_hll_build(int log_p, const DevCsr &B, uint8_t *hll, hipStream_t s) {
 }
 
 __device__ __forceinline__ uint32_t bytemax4(uint32_t a, uint32_t b) {
-  uint32_t r = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t x = (a >> (8 * i)) & 255u, y = (b >> (8 * i)) & 255u;
-    r |= (x > y ? x : y) << (8 * i);
-  }
-  return r;
+  // two bytes in each half word, so a 16-bit maximum per half is theirs
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  auto half_max = [](uint32_t x, uint32_t y) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, x),
+                                                                  __builtin_bit_cast(us2, y)));
+  };
+  return half_max(a & 0x00FF00FFu, b & 0x00FF00FFu) |
+         half_max((a >> 8) & 0x00FF00FFu, (b >> 8) & 0x00FF00FFu) << 8;
 }
 
 struct HllConst {
@@ -727,12 +772,12 @@ __device__ __forceinline__ int32_t hll_estimate_wave(uint32_t m, const HllConst 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint32_t b = (m >> (8 * i)) & 255u;
-      z += 1.0 / (double)(1ull << b);
+      z += __longlong_as_double((long long)(1023u - b) << 52);  // 2^-b, b <= 33
       empty += b == 0;
     }
   }
-  z = group_sum(z, kWave);
-  empty = group_sum(empty, kWave);
+  z = group_sum(z, W);  // the other lanes hold zeros
+  empty = group_sum(empty, W);
   constexpr double alpha = LOGP == 5 ? 0.697 : 0.709;  // HLL_CONSTANT
   int32_t result = (int32_t)(alpha * P * P / z);
   if (empty != 0 && result < 2.5 * P) result = hc.lc[empty];
@@ -752,10 +797,22 @@ __device__ __forceinline__ uint32_t hll_merge_range(const uint32_t *a_ci,
   constexpr int W = P / 4;     // words per sketch
   constexpr int S = kWave / W; // sketches per step
   const int sk = lane / W, w = lane % W;
+  // eight gathers in flight (one at a time, each behind the load of its
+  // column, a sampled row of 2000 entries took 53 us); an entry past the end
+  // reads nothing and is the neutral 0
+  constexpr int U = 8;
   uint32_t m = 0;
-  for (uint32_t j = s + sk; j < e; j += S) {
-    const uint32_t k = a_ci[j];
-    m = bytemax4(m, reinterpret_cast<const uint32_t *>(hll + (uint64_t)k * P)[w]);
+  for (uint32_t j = s + sk; j < e; j += U * S) {
+    uint32_t k[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) k[u] = e - j > (uint32_t)(u * S) ? a_ci[j + u * S] : 0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = e - j > (uint32_t)(u * S)
+                 ? reinterpret_cast<const uint32_t *>(hll + (uint64_t)k[u] * P)[w]
+                 : 0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) m = bytemax4(m, v[u]);
   }
   for (int d = W; d < kWave; d <<= 1) m = bytemax4(m, __shfl_xor(m, d));
   return m;
@@ -882,9 +939,9 @@ int launch_hll_merge(int log_p, const DevCsr &A, const uint8_t *hll,
   std::memcpy(hc.num_sizes, tables().hash_num, sizeof(hc.num_sizes));
   uint32_t *heavy_count = (uint32_t *)temp;
   uint32_t *heavy_list = heavy_count + 16;
-  HIP_TRY(hipMemsetAsync(heavy_count, 0, 4, s));
+  OC_TRY(launch_fill_u32(heavy_count, 1, 0u, s));
   const uint32_t rows = (uint32_t)A.rows;
-  const uint32_t heavy = 2048;
+  const uint32_t heavy = 512;  // entries one wave merges
   const uint32_t ntasks = mode == 0 ? rows : nsamples;
   dim3 grid(std::max<uint32_t>(1, std::min<uint32_t>(cdiv(ntasks, 4), 1u << 18)));
   dim3 hgrid(std::max<uint32_t>(1, tables().num_cu));
