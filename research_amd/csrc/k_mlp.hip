@@ -203,6 +203,7 @@ __device__ void stage_x_wave(MlpSmem &s, const float *__restrict__ feat, uint64_
 __device__ f4 forward_wave(MlpSmem &s, int r0) {
   const int l = lane_id();
   const int col = l & 15, rb = (l >> 4) * 4;
+#pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = mfma(ld_rowk(s.X, kS32, r0, 0), ld_rowk(s.W1t, kS32, nt * 16, 0), acc);
@@ -212,6 +213,7 @@ __device__ f4 forward_wave(MlpSmem &s, int r0) {
       s.H1[(r0 + rb + r) * kS64 + nt * 16 + col] = f2bf(relu(acc[r] + bb));
   }
   wave_sync();
+#pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = mfma(ld_rowk(s.H1, kS64, r0, 0), ld_rowk(s.W2t, kS64, nt * 16, 0), acc);
@@ -230,20 +232,28 @@ __device__ f4 forward_wave(MlpSmem &s, int r0) {
   return z;
 }
 
+// The value of lane ^ 1, lane ^ 2 and, once quads agree, of the other quad of
+// eight lanes: DPP moves, without the LDS round trip of a shuffle.
+template <int CTRL>
+__device__ inline float dpp_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppOtherQuad = 0x141;
+
 // Softmax over the 8 class lanes of each row group (lanes with l%16 >= 8
 // carry padding and compute values nobody reads).
 __device__ inline void softmax8(float z, float &p, float &m, float &sum) {
   const bool valid = (lane_id() & 15) < kC;
   float zz = valid ? z : -1e30f;
   m = zz;
-  m = fmaxf(m, __shfl_xor(m, 1));
-  m = fmaxf(m, __shfl_xor(m, 2));
-  m = fmaxf(m, __shfl_xor(m, 4));
+  m = fmaxf(m, dpp_f<kDppXor1>(m));
+  m = fmaxf(m, dpp_f<kDppXor2>(m));
+  m = fmaxf(m, dpp_f<kDppOtherQuad>(m));
   const float e = valid ? expf(zz - m) : 0.f;
   sum = e;
-  sum += __shfl_xor(sum, 1);
-  sum += __shfl_xor(sum, 2);
-  sum += __shfl_xor(sum, 4);
+  sum += dpp_f<kDppXor1>(sum);
+  sum += dpp_f<kDppXor2>(sum);
+  sum += dpp_f<kDppOtherQuad>(sum);
   p = e / sum;
 }
 
@@ -346,6 +356,7 @@ __global__ __launch_bounds__(kMlpBlock) void k_mlp_backward(
   }
   wave_sync();
   // dZ2 = (dZ3 W3^T) * [H2 > 0]
+#pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = mfma(ld_rowk(sb.dZ3, kS32, r0, 0), ld_rowk(sb.W3h, kS32, nt * 16, 0), acc);
@@ -357,6 +368,7 @@ __global__ __launch_bounds__(kMlpBlock) void k_mlp_backward(
   }
   wave_sync();
   // dZ1 = (dZ2 W2^T) * [H1 > 0]
+#pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = mfma(ld_rowk(sb.dZ2, kS64, r0, 0), ld_rowk(sb.W2n, kS64, nt * 16, 0), acc);
@@ -372,7 +384,8 @@ __global__ __launch_bounds__(kMlpBlock) void k_mlp_backward(
   float *out = partial + (uint64_t)blockIdx.x * kNParam;
   {  // dW2[h1][h2]: wave w takes h1 tile w
     const int mt = w;
-    for (int nt = 0; nt < 4; ++nt) {
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
       acc = mfma(ld_colk(s.H1, kS64, mt * 16, 0), ld_colk(sb.dZ2, kS64, nt * 16, 0), acc);
       acc = mfma(ld_colk(s.H1, kS64, mt * 16, 32), ld_colk(sb.dZ2, kS64, nt * 16, 32), acc);
