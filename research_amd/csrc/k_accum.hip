@@ -952,8 +952,10 @@ __device__ __forceinline__ void for_bucket(const uint32_t *ck, uint32_t s0, uint
 // many products meet in one output, which these rows, bounded by their
 // products, do not have room for.  Returns false, having written nothing,
 // for a row it does not take: the table's path follows.  (85,720 Erdos-Renyi
-// rows of 576 products: 684 -> @SR1@ us; R-MAT 2^18's rows of the largest
-// tables: 1411 -> @SR2@ us.)
+// rows of 576 products: 684 -> 417 us.)  Tables of 1024 threads are not
+// taken: their rows come from skewed structures that crowd the buckets and
+// need U = 12, 121 registers a lane; R-MAT 2^18's took 2324 us so, 1288 by
+// the table.
 //
 // LDS: header, bucket starts and duplicate counts (u16, 4 BS each), then the
 // products' columns and values in bucket order.
@@ -1415,7 +1417,6 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
   if (o.nnz && threadIdx.x == 0) o.nnz[r] = n;
 }
 
-// (eight waves per SIMD: the bins fill the CU's waves)
 template <int BS, typename T, bool EST>
 __global__ __launch_bounds__(BS) void k_num_hash(KArgs<T> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, const uint32_t *__restrict__ err, HashLayout L, KOut<T> o, int key_bits,
