@@ -423,24 +423,43 @@ int launch_analysis(const DevCsr &A, const DevCsr &B, const RowInfo &ri,
 // Copies a few device words into a pinned host page and then sets the page's
 // flag, on which the host spins.  A copy into pageable memory and a stream
 // synchronisation took 12 us more for each value the host waits for.
-__global__ __launch_bounds__(1024) void k_publish(PublishArgs pa, uint32_t *dst, uint32_t *flag,
-                                                  uint32_t seq) {
+__global__ __launch_bounds__(1024) void k_publish(PublishTo to) {
   uint32_t at = 0;
   for (int k = 0; k < PublishArgs::kMax; ++k) {
-    for (uint32_t i = threadIdx.x; i < pa.words[k]; i += blockDim.x) dst[at + i] = pa.src[k][i];
-    at += pa.words[k];
+    for (uint32_t i = threadIdx.x; i < to.pa.words[k]; i += blockDim.x)
+      to.dst[at + i] = to.pa.src[k][i];
+    at += to.pa.words[k];
   }
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0)
-    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(to.flag, to.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-int launch_publish(const PublishArgs &pa, uint32_t *dst, uint32_t *flag, uint32_t seq,
-                   hipStream_t s) {
+// The same at the end of the kernel that produces the last of the words: the
+// scans' totals and the bins' offsets are what the host waits for most, and a
+// launch less is about 5 us of a small product.  Called by all threads of one
+// workgroup, whose first wave copies what it and earlier launches wrote.
+__device__ void publish_here(const PublishTo &to) {
+  if (!to.flag) return;
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  uint32_t at = 0;
+  for (int k = 0; k < PublishArgs::kMax; ++k) {
+    for (uint32_t i = threadIdx.x; i < to.pa.words[k]; i += kWave)
+      to.dst[at + i] = to.pa.src[k][i];
+    at += to.pa.words[k];
+  }
+  __threadfence_system();  // every lane's words, before the flag
+  __builtin_amdgcn_wave_barrier();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(to.flag, to.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int launch_publish(const PublishTo &to, hipStream_t s) {
   uint32_t most = 0;
-  for (int k = 0; k < PublishArgs::kMax; ++k) most = std::max(most, pa.words[k]);
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(most > 64 ? 1024 : 64), 0, s, pa, dst, flag, seq);
+  for (int k = 0; k < PublishArgs::kMax; ++k) most = std::max(most, to.pa.words[k]);
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(most > 64 ? 1024 : 64), 0, s, to);
   LAUNCH_CHECK();
   return OC_OK;
 }
@@ -466,7 +485,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_partials(
-    uint64_t *part, uint32_t nparts, uint64_t *total_out) {
+    uint64_t *part, uint32_t nparts, uint64_t *total_out, PublishTo to) {
   __shared__ uint64_t sc[17];
   uint64_t carry = 0;
   for (uint32_t b0 = 0; b0 < nparts; b0 += kScanBlock) {
@@ -478,11 +497,12 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_partials(
     carry += tot;
   }
   if (threadIdx.x == 0) *total_out = carry;
+  publish_here(to);
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_final(
-    const uint32_t *__restrict__ in, uint64_t *__restrict__ out, uint64_t n,
-    const uint64_t *__restrict__ part, int write_total) {
+    const uint32_t *__restrict__ in, uint64_t *out, uint64_t n,
+    const uint64_t *__restrict__ part, int write_total, PublishTo to) {
   __shared__ uint64_t sc[17];
   const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
@@ -499,7 +519,10 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_final(
     if (base + i < n) out[base + i] = run;
     run += v[i];
   }
-  if (write_total && threadIdx.x == 0) out[n] = tot;
+  if (write_total) {
+    if (threadIdx.x == 0) out[n] = tot;
+    publish_here(to);
+  }
 }
 
 // Two launches for the row counts of most products: smaller tiles (more
@@ -551,8 +574,8 @@ __global__ __launch_bounds__(kScan2Block) void k_scan2_reduce(
 
 template <bool VEC>
 __global__ __launch_bounds__(kScan2Block) void k_scan2_final(
-    const uint32_t *__restrict__ in, uint64_t *__restrict__ out, uint64_t n,
-    const uint64_t *__restrict__ part) {
+    const uint32_t *__restrict__ in, uint64_t *out, uint64_t n,
+    const uint64_t *__restrict__ part, PublishTo to) {
   __shared__ uint64_t sc[4], sw[4];
   const uint64_t base = (uint64_t)blockIdx.x * kScan2Tile + threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
@@ -584,6 +607,7 @@ __global__ __launch_bounds__(kScan2Block) void k_scan2_final(
   }
   // the thread whose items hold the last one
   if (base < n && base + kScanItems >= n) out[n] = run;
+  if (blockIdx.x == gridDim.x - 1) publish_here(to);
 }
 
 static bool scan2(uint64_t n) { return n > kScanTile && n <= (uint64_t)kScan2Tile * kScan2Tiles; }
@@ -594,17 +618,17 @@ size_t scan_temp_bytes(uint64_t n) {
 }
 
 int launch_scan_u32(const uint32_t *in, uint64_t *out, uint64_t n, void *temp,
-                    hipStream_t s) {
+                    hipStream_t s, const PublishTo &to) {
   if (n == 0) {  // out[0] = 0 by a kernel, not a memset node (capture-safe)
     hipLaunchKernelGGL(k_scan_final, dim3(1), dim3(kScanBlock), 0, s, in, out,
-                       (uint64_t)0, (const uint64_t *)nullptr, 1);
+                       (uint64_t)0, (const uint64_t *)nullptr, 1, to);
     LAUNCH_CHECK();
     return OC_OK;
   }
   uint32_t nb = cdiv(n, kScanTile);
   if (nb == 1) {
     hipLaunchKernelGGL(k_scan_final, dim3(1), dim3(kScanBlock), 0, s, in, out,
-                       n, (const uint64_t *)nullptr, 1);
+                       n, (const uint64_t *)nullptr, 1, to);
     LAUNCH_CHECK();
     return OC_OK;
   }
@@ -617,20 +641,20 @@ int launch_scan_u32(const uint32_t *in, uint64_t *out, uint64_t n, void *temp,
     LAUNCH_CHECK();
     if (vec)
       hipLaunchKernelGGL(k_scan2_final<true>, dim3(nt), dim3(kScan2Block), 0, s, in, out, n,
-                         (const uint64_t *)part);
+                         (const uint64_t *)part, to);
     else
       hipLaunchKernelGGL(k_scan2_final<false>, dim3(nt), dim3(kScan2Block), 0, s, in, out, n,
-                         (const uint64_t *)part);
+                         (const uint64_t *)part, to);
     LAUNCH_CHECK();
     return OC_OK;
   }
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanBlock), 0, s, in, n, part);
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kScanBlock), 0, s, part, nb,
-                     out + n);
+                     out + n, to);
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(kScanBlock), 0, s, in, out, n,
-                     (const uint64_t *)part, 0);
+                     (const uint64_t *)part, 0, PublishTo{});
   LAUNCH_CHECK();
   return OC_OK;
 }
@@ -1106,7 +1130,7 @@ __global__ __launch_bounds__(kBinBlock) void k_bin_classify(
 // another took 22 us of barriers at 391 blocks and 153 us at 6008; now 3
 // and 16.
 __global__ __launch_bounds__(1024) void k_bin_scan(uint32_t *__restrict__ hist, uint32_t nblocks,
-                                                   uint32_t *__restrict__ bin_offsets) {
+                                                   uint32_t *bin_offsets, PublishTo to) {
   constexpr int U = 8;
   static_assert(kBinSlots <= 1024 / kWave, "a wave for each bin");
   __shared__ uint32_t tot[1024 / kWave];
@@ -1146,6 +1170,7 @@ __global__ __launch_bounds__(1024) void k_bin_scan(uint32_t *__restrict__ hist, 
     for (uint32_t q = 0; q < threadIdx.x; ++q) run += tot[q];
     bin_offsets[threadIdx.x] = run;
   }
+  publish_here(to);  // the rows' scatter need not be done
 }
 
 __global__ __launch_bounds__(kBinBlock) void k_bin_scatter(
@@ -1182,7 +1207,7 @@ size_t bin_temp_bytes(uint64_t rows) {
 
 int launch_binning(const BinParams &bp, uint64_t rows, uint8_t *bin_of_row,
                    uint32_t *bin_rows, uint32_t *bin_offsets, void *temp,
-                   hipStream_t s) {
+                   hipStream_t s, const PublishTo &to) {
   const Tables &t = tables();
   BinTables bt;
   std::memcpy(bt.hash_sym, t.hash_sym, sizeof(bt.hash_sym));
@@ -1209,7 +1234,7 @@ int launch_binning(const BinParams &bp, uint64_t rows, uint8_t *bin_of_row,
   ba.skip_flag = bp.skip_flag;
   if (rows == 0) {
     HIP_TRY(hipMemsetAsync(bin_offsets, 0, 4 * (kBinSlots + 1), s));
-    return OC_OK;
+    return to.flag ? launch_publish(to, s) : OC_OK;
   }
   const uint32_t nb = cdiv(rows, kBinBlock);
   uint32_t *hist = (uint32_t *)temp;
@@ -1226,7 +1251,7 @@ int launch_binning(const BinParams &bp, uint64_t rows, uint8_t *bin_of_row,
   hipLaunchKernelGGL(k_bin_classify, dim3(nb), dim3(kBinBlock), 0, s, ba, bt,
                      (uint32_t)rows, bin_of_row, hist);
   LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, hist, nb, bin_offsets);
+  hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, s, hist, nb, bin_offsets, to);
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_bin_scatter, dim3(nb), dim3(kBinBlock), 0, s,
                      (const uint8_t *)bin_of_row, (uint32_t)rows,

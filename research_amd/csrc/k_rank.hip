@@ -645,13 +645,13 @@ __global__ __launch_bounds__(256) void k_bm_mark(const uint32_t *__restrict__ sz
 int launch_bitmap_offsets(const uint8_t *bin_of_row, int bin_lo, int bin_hi, uint64_t m,
                           const uint32_t *products, const uint32_t *left,
                           const uint32_t *right, uint32_t min_products, uint32_t *sz,
-                          void *scan_tmp, uint64_t *bmoff, hipStream_t s) {
+                          void *scan_tmp, uint64_t *bmoff, hipStream_t s, const PublishTo &to) {
   if (m) {
     hipLaunchKernelGGL(k_bm_sizes, dim3(cdiv(m, 256)), dim3(256), 0, s, bin_of_row, bin_lo,
                        bin_hi, (uint32_t)m, products, left, right, min_products, sz);
     LAUNCH_CHECK();
   }
-  OC_TRY(launch_scan_u32(sz, bmoff, m, scan_tmp, s));
+  OC_TRY(launch_scan_u32(sz, bmoff, m, scan_tmp, s, to));
   if (m) {
     hipLaunchKernelGGL(k_bm_mark, dim3(cdiv(m, 256)), dim3(256), 0, s, (const uint32_t *)sz,
                        (uint32_t)m, bmoff);

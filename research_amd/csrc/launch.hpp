@@ -76,8 +76,14 @@ struct PublishArgs {
   const uint32_t *src[kMax] = {nullptr, nullptr, nullptr};
   uint32_t words[kMax] = {0, 0, 0};
 };
-int launch_publish(const PublishArgs &pa, uint32_t *dst, uint32_t *flag, uint32_t seq,
-                   hipStream_t s);
+// A publish by the kernel that produces the last of the words instead of a
+// launch of its own (one wave copies, so a few words only).
+struct PublishTo {
+  PublishArgs pa;
+  uint32_t *dst = nullptr, *flag = nullptr;  // null: nothing to publish
+  uint32_t seq = 0;
+};
+int launch_publish(const PublishTo &to, hipStream_t s);
 // bounds = {0, *count}: the row range of a device-counted list
 int launch_count_bounds(const uint32_t *count, uint32_t *bounds, hipStream_t s);
 size_t scan_temp_bytes(uint64_t n);
@@ -85,7 +91,7 @@ size_t scan_temp_bytes(uint64_t n);
 // oc_analysis_noalloc counts this)
 size_t scan_temp_bytes_min(uint64_t n);
 int launch_scan_u32(const uint32_t *in, uint64_t *out, uint64_t n, void *temp,
-                    hipStream_t s);
+                    hipStream_t s, const PublishTo &to = PublishTo{});
 int launch_murmur(const uint32_t *cols, uint32_t *out, uint64_t n,
                   hipStream_t s);
 int launch_hll_build(int log_p, const DevCsr &B, uint8_t *hll, hipStream_t s);
@@ -116,7 +122,7 @@ struct BinParams {
 size_t bin_temp_bytes(uint64_t rows);
 int launch_binning(const BinParams &bp, uint64_t rows, uint8_t *bin_of_row,
                    uint32_t *bin_rows, uint32_t *bin_offsets, void *temp,
-                   hipStream_t s);
+                   hipStream_t s, const PublishTo &to = PublishTo{});
 
 // Copy rows (all rows, or those listed) from a temp layout into C.
 // A row whose count exceeds cap[row] (when cap is given) is skipped.
@@ -265,7 +271,8 @@ int launch_num_rank1(const AccArgs &a, const uint32_t *rows, uint32_t nrows, uin
 int launch_bitmap_offsets(const uint8_t *bin_of_row, int bin_lo, int bin_hi, uint64_t m,
                           const uint32_t *products, const uint32_t *left,
                           const uint32_t *right, uint32_t min_products, uint32_t *sz,
-                          void *scan_tmp, uint64_t *bmoff, hipStream_t s);
+                          void *scan_tmp, uint64_t *bmoff, hipStream_t s,
+                          const PublishTo &to = PublishTo{});
 // Ultra-sparse expand-sort-compress for all rows with products <= esc_n.
 int launch_esc(int esc_n, const AccArgs &a, const NumOut &o, hipStream_t s);
 

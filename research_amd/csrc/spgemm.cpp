@@ -528,17 +528,18 @@ struct Run {
 
   // ------------------------------------------------ values for the host
   // publish() queues a copy of a few device words to the handle's pinned
-  // page; await() waits for the latest one and returns them.  The wait spins
-  // on the page's flag, and after 200 us synchronises with the stream
-  // instead, which also reports a failed launch.
+  // page (target(): by a kernel that the caller launches next); await() waits
+  // for the latest one and returns them.  The wait spins on the page's flag,
+  // and after 200 us synchronises with the stream instead, which also reports
+  // a failed launch.
   struct Words {
     const void *dev;
     uint32_t n;
   };
-  int publish(std::initializer_list<Words> w) {
+  int target(std::initializer_list<Words> w, PublishTo *to) {
     HostPage &pg = h->page;
     HIP_TRY(pg.take());
-    PublishArgs pa;
+    PublishArgs &pa = to->pa;
     int k = 0;
     uint32_t total = 0;
     for (const Words &x : w) {
@@ -549,7 +550,15 @@ struct Run {
     }
     OC_REQUIRE(total <= HostPage::kWords - HostPage::kData, "internal: a host read of %u words",
                total);
-    return launch_publish(pa, pg.p + HostPage::kData, pg.p, ++pg.seq, s);
+    to->dst = pg.p + HostPage::kData;
+    to->flag = pg.p;
+    to->seq = ++pg.seq;
+    return OC_OK;
+  }
+  int publish(std::initializer_list<Words> w) {
+    PublishTo to;
+    OC_TRY(target(w, &to));
+    return launch_publish(to, s);
   }
   int await(const uint32_t **out) {
     HostPage &pg = h->page;
@@ -639,16 +648,20 @@ struct Run {
   // together with the bitmaps' size.
   static constexpr uint32_t kBitmapMinProducts = 2048;
   uint64_t *bmoff_all = nullptr;
-  int bitmap_offsets(const uint8_t *bor) {
+  bool want_bitmaps() {
     h->bitmap_bytes = 0;
     const bool blocks = h->b_block_base != nullptr && h->b_block_rp == (const void *)B.rp;
-    if (h->cfg.use_tiled_numeric != 3 || blocks || h->max_products < kBitmapMinProducts)
-      return OC_OK;
+    return h->cfg.use_tiled_numeric == 3 && !blocks && h->max_products >= kBitmapMinProducts;
+  }
+  // publishes the bin offsets (boff) and the bitmaps' size
+  int bitmap_offsets(const uint8_t *bor, const uint32_t *boff) {
     uint32_t *sz;
     OC_TRY(ar.get(&bmoff_all, A.rows + 1));
     OC_TRY(ar.get(&sz, A.rows));
+    PublishTo to;
+    OC_TRY(target({{boff, kBinSlots + 1}, {bmoff_all + A.rows, 2}}, &to));
     return launch_bitmap_offsets(bor, 6, 14, A.rows, ri.products, ri.left, ri.right,
-                                 kBitmapMinProducts, sz, scan_tmp, bmoff_all, s);
+                                 kBitmapMinProducts, sz, scan_tmp, bmoff_all, s, to);
   }
   int row_bitmaps(uint64_t n4) {
     if (n4 == 0 || (double)n4 * 16 > 0.2 * (double)h->dev_bytes) return OC_OK;
@@ -713,7 +726,8 @@ struct Run {
 
   // C: u64 offsets (rows+1) from per-row counts, then (once the host has
   // read offsets[rows]) cols/values.
-  int c_offsets(const uint32_t *nnz) {
+  // `also`: published with C's size (nothing is when null)
+  int c_offsets(const uint32_t *nnz, const Words *also = nullptr) {
     const uint64_t m = A.rows;
     if (!C->row_offsets) {
       C->rows = m;
@@ -724,7 +738,9 @@ struct Run {
       C->owned = 3;  // output cache (out_alloc)
       OC_TRY(out_alloc(&C->row_offsets, (m + 1) * 8));
     }
-    return launch_scan_u32(nnz, (uint64_t *)C->row_offsets, m, scan_tmp, s);
+    PublishTo to;
+    if (also) OC_TRY(target({c_nnz(), *also}, &to));
+    return launch_scan_u32(nnz, (uint64_t *)C->row_offsets, m, scan_tmp, s, to);
   }
   Words c_nnz() const { return Words{(const uint64_t *)C->row_offsets + A.rows, 2}; }
   int c_entries(uint64_t nnzc) {
@@ -736,7 +752,10 @@ struct Run {
   }
 
   // Queues the binning; the caller reads the bin offsets (boff).
-  int queue_binning(const BinParams &bp, uint8_t **bor, uint32_t **brows, uint32_t **boff) {
+  // With `pub`, the bin offsets are published, before or after those words.
+  int queue_binning(const BinParams &bp, uint8_t **bor, uint32_t **brows, uint32_t **boff,
+                    bool pub = false, Words first = Words{nullptr, 0},
+                    Words last = Words{nullptr, 0}) {
     const uint64_t m = A.rows;
     if (!*bor) {
       OC_TRY(ar.get(bor, m));
@@ -746,7 +765,9 @@ struct Run {
     uint8_t *tmp;
     OC_TRY(ar.get(&tmp, bin_temp_bytes(m)));
     bin_tmp = tmp;
-    return launch_binning(bp, m, *bor, *brows, *boff, tmp, s);
+    PublishTo to;
+    if (pub) OC_TRY(target({first, {*boff, kBinSlots + 1}, last}, &to));
+    return launch_binning(bp, m, *bor, *brows, *boff, tmp, s, to);
   }
 
   // Select the long rows for the band kernels and build their tables.
@@ -900,10 +921,12 @@ int Run::prologue_and_analysis() {
   // keeps it for whole-path replays
   if (!h->keep_plan) ar.free(atmp);
   mk.mark("analysis_product_calc");
-  OC_TRY(launch_scan_u32(ri.products, psum_prod, m, scan_tmp, s));
-  mk.mark("analysis_reduce");
   const uint32_t *w;
-  OC_TRY(fetch({{scal, 2}, {psum_prod + m, 2}}, &w));
+  PublishTo to;
+  OC_TRY(target({{scal, 2}, {psum_prod + m, 2}}, &to));
+  OC_TRY(launch_scan_u32(ri.products, psum_prod, m, scan_tmp, s, to));
+  mk.mark("analysis_reduce");
+  OC_TRY(await(&w));
   h->max_a_nnz = w[0];
   h->max_products = w[1];
   h->total_products = u64_at(w + 2);
@@ -964,9 +987,11 @@ int Run::learned_capacities(bool *use_est) {
   ar.free(feat);
   uint64_t *ps;
   OC_TRY(ar.get(&ps, m + 1));
-  OC_TRY(launch_scan_u32(learned_est, ps, m, scan_tmp, s));
   const uint32_t *w;
-  OC_TRY(fetch({{ps + m, 2}}, &w));
+  PublishTo to;
+  OC_TRY(target({{ps + m, 2}}, &to));
+  OC_TRY(launch_scan_u32(learned_est, ps, m, scan_tmp, s, to));
+  OC_TRY(await(&w));
   h->learned_total = u64_at(w);
   ar.free(ps);
   h->learned_consulted = true;
@@ -1153,10 +1178,11 @@ int Run::run_fat() {
   OC_TRY(launch_fat_count(bits, m, B.cols, nnz, s));
   fam("fat", "numeric_fat", true, nullptr, (uint32_t)m);
   mk.mark("numeric_fat");
-  OC_TRY(c_offsets(nnz));
-  mk.mark("epilogue_scan");
   const uint32_t *w;
-  OC_TRY(fetch({c_nnz()}, &w));
+  const Words nothing{nullptr, 0};
+  OC_TRY(c_offsets(nnz, &nothing));
+  mk.mark("epilogue_scan");
+  OC_TRY(await(&w));
   OC_TRY(c_entries(u64_at(w)));
   OC_TRY(launch_fat_compact(A.vtype, dense, bits, m, B.cols, (const uint64_t *)C->row_offsets,
                             C->col_ids, C->values, s));
@@ -1200,17 +1226,18 @@ int Run::run_usparse() {
     uint8_t *bor = nullptr;
     uint32_t *brows = nullptr, *boff = nullptr;
     uint32_t hoff[kBinSlots + 1];
-    OC_TRY(queue_binning(bp, &bor, &brows, &boff));
-    OC_TRY(fetch({{boff, kBinSlots + 1}}, &w));
+    OC_TRY(queue_binning(bp, &bor, &brows, &boff, true));
+    OC_TRY(await(&w));
     std::memcpy(hoff, w, sizeof(hoff));
     std::memcpy(h->bin2, hoff, sizeof(hoff));
     h->have_bin2 = true;
     OC_TRY(numeric_bins(brows, hoff, o, true, boff));
     mk.mark("numeric_usparse_outlier");
   }
-  OC_TRY(c_offsets(nnz));
+  const Words listed{ovf, ovf ? 1u : 0u};
+  OC_TRY(c_offsets(nnz, &listed));
   mk.mark("epilogue_scan");
-  OC_TRY(fetch({c_nnz(), {ovf, ovf ? 1u : 0u}}, &w));
+  OC_TRY(await(&w));
   if (ovf && w[2]) {
     set_error("internal: %u ultra-sparse outlier rows overflowed", w[2]);
     return OC_ERR_CAPACITY;
@@ -1243,17 +1270,17 @@ int Run::run_precise() {
   uint32_t *brows = nullptr, *boff = nullptr;
   uint32_t hoff[kBinSlots + 1];
   const uint32_t *w;
-  OC_TRY(queue_binning(bp, &bor, &brows, &boff));
-  OC_TRY(bitmap_offsets(bor));
+  const bool bitmaps = want_bitmaps();
+  OC_TRY(queue_binning(bp, &bor, &brows, &boff, !bitmaps));
+  if (bitmaps) OC_TRY(bitmap_offsets(bor, boff));
   mk.mark("symbolic_binning");
-  OC_TRY(fetch({{boff, kBinSlots + 1}, {bmoff_all ? bmoff_all + m : nullptr, bmoff_all ? 2u : 0u}},
-               &w));
+  OC_TRY(await(&w));
   std::memcpy(hoff, w, sizeof(hoff));
   std::memcpy(h->bin1, hoff, sizeof(hoff));
   h->have_bin1 = true;
   const AccArgs a = acc();
   const Tables &t = tables();
-  if (bmoff_all) OC_TRY(row_bitmaps(u64_at(w + kBinSlots + 1)));
+  if (bitmaps) OC_TRY(row_bitmaps(u64_at(w + kBinSlots + 1)));
   auto stage = [&](const char *name, bool work) {
     if (work) mk.mark(name);
     else mk.none(name);
@@ -1307,9 +1334,9 @@ int Run::run_precise() {
   auto counted = [&]() -> int {
     OC_TRY(c_offsets(nnz));
     mk.mark("epilogue_scan");
-    OC_TRY(queue_binning(nb, &bor2, &brows2, &boff2));
+    OC_TRY(queue_binning(nb, &bor2, &brows2, &boff2, true, c_nnz(), Words{ovf, 1}));
     mk.mark("numeric_binning");
-    return fetch({c_nnz(), {boff2, kBinSlots + 1}, {ovf, 1}}, &w);
+    return await(&w);
   };
   OC_TRY(counted());
   h->sym_overflow_rows = w[2 + kBinSlots + 1];
@@ -1458,9 +1485,11 @@ int Run::run_est() {
   OC_TRY(queue_binning(bp, &bor, &brows, &boff));
   uint64_t *psum_est;
   OC_TRY(ar.get(&psum_est, m + 1));
-  OC_TRY(launch_scan_u32(est, psum_est, m, scan_tmp, s));
+  PublishTo to;
+  OC_TRY(target({{boff, kBinSlots + 1}, {psum_est + m, 2}}, &to));
+  OC_TRY(launch_scan_u32(est, psum_est, m, scan_tmp, s, to));
   mk.mark("numeric_binning");
-  OC_TRY(fetch({{boff, kBinSlots + 1}, {psum_est + m, 2}}, &w));
+  OC_TRY(await(&w));
   std::memcpy(hoff, w, sizeof(hoff));
   std::memcpy(h->bin2, hoff, sizeof(hoff));
   h->have_bin2 = true;
@@ -1511,9 +1540,10 @@ int Run::run_est() {
   // C's offsets are queued as if no row had outgrown its slot; the host
   // reads C's size together with the overflow count
   auto counted = [&]() -> int {
-    OC_TRY(c_offsets(nnz));
+    const Words over{ovf, 1};
+    OC_TRY(c_offsets(nnz, &over));
     mk.mark("epilogue_scan");
-    return fetch({c_nnz(), {ovf, 1}}, &w);
+    return await(&w);
   };
   OC_TRY(counted());
   const uint32_t n1 = w[2];
