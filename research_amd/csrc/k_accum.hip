@@ -1678,31 +1678,65 @@ __global__ __launch_bounds__(kWinBlock) void k_window(
 // Column tiles of W = 2^logW columns.  ts[k * T1 + t] is the index of the
 // first entry of B row k whose column is >= t * W (T1 = tiles + 1), so the
 // part of any B row inside any tile is known without walking the row.
-// A wave takes 64 / P rows at once, P = 2^logP lanes per row (T1 rounded up
-// to a power of two, at most 64), so narrow tables keep every lane busy.
-__global__ __launch_bounds__(256) void k_tile_starts(const uint32_t *__restrict__ b_rp,
-                                                     const uint32_t *__restrict__ b_ci,
-                                                     uint32_t rows, uint32_t logW,
-                                                     uint32_t T1, const uint32_t *__restrict__ base,
-                                                     uint32_t *__restrict__ ts, uint32_t logP) {
-  const uint32_t lane = (uint32_t)lane_id(), P = 1u << logP, sub = lane >> logP;
-  const uint32_t per_wave = kWave >> logP;
-  const uint32_t waves = gridDim.x * 4;
-  for (uint32_t k0 = (blockIdx.x * 4 + threadIdx.x / kWave) * per_wave; k0 < rows;
-       k0 += waves * per_wave) {
-    const uint32_t k = k0 + sub;
-    if (k >= rows) continue;
-    const uint32_t s = b_rp[k], e = b_rp[k + 1];
-    const uint64_t b0 = base ? base[k] : 0;  // tiles counted from the row's block
-    for (uint32_t t = lane & (P - 1); t < T1; t += P) {
-      const uint64_t bound = b0 + ((uint64_t)t << logW);
-      uint32_t lo = s, hi = e;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if ((uint64_t)b_ci[mid] < bound) lo = mid + 1;
-        else hi = mid;
+// The table's entries are spread over the lanes in memory order, kTsItems to
+// each: the writes are whole lines whatever T1 is, and the searches of one
+// lane, each a chain of dependent loads, run side by side.  A wave for each
+// row waited out one chain at a time, twice where T1 is just over 64, and
+// took a workgroup for every four rows.  (2^20 rows of 16 entries: 65
+// starts each 514 -> 193 us, 9 each 110 -> 39; 1.5 million rows of a batch in
+// one or two tiles each 42 -> 29 a launch.)
+constexpr int kTsItems = 4, kTsBlock = 256;
+constexpr uint32_t kTsTile = kTsBlock * kTsItems;
+__global__ __launch_bounds__(kTsBlock) void k_tile_starts(const uint32_t *__restrict__ b_rp,
+                                                          const uint32_t *__restrict__ b_ci,
+                                                          uint64_t total, uint32_t logW,
+                                                          uint32_t T1,
+                                                          const uint32_t *__restrict__ base,
+                                                          uint32_t *__restrict__ ts) {
+  for (uint64_t i0 = (uint64_t)blockIdx.x * kTsTile; i0 < total;
+       i0 += (uint64_t)gridDim.x * kTsTile) {
+    const uint32_t k0 = (uint32_t)(i0 / T1), t0 = (uint32_t)(i0 - (uint64_t)k0 * T1);
+    uint32_t lo[kTsItems], hi[kTsItems];
+    uint64_t bound[kTsItems];
+#pragma unroll
+    for (int u = 0; u < kTsItems; ++u) {
+      const uint32_t j = u * kTsBlock + threadIdx.x;
+      lo[u] = hi[u] = 0;
+      bound[u] = 0;
+      if (i0 + j < total) {
+        const uint32_t q = t0 + j, dk = q / T1, k = k0 + dk;
+        lo[u] = b_rp[k];
+        hi[u] = b_rp[k + 1];
+        const uint32_t t = q - dk * T1;
+        // tiles counted from the row's block; the first and the last entry,
+        // half of a narrow table, are the row's ends and need no search
+        bound[u] = (base ? base[k] : 0) + ((uint64_t)t << logW);
+        if (t == 0) hi[u] = lo[u];
+        else if (t == T1 - 1) lo[u] = hi[u];
       }
-      ts[(uint64_t)k * T1 + t] = lo;
+    }
+    for (;;) {
+      bool more = false;
+#pragma unroll
+      for (int u = 0; u < kTsItems; ++u) more |= lo[u] < hi[u];
+      if (!more) break;
+      uint32_t c[kTsItems], mid[kTsItems];
+#pragma unroll
+      for (int u = 0; u < kTsItems; ++u) {
+        mid[u] = (lo[u] + hi[u]) >> 1;
+        c[u] = b_ci[lo[u] < hi[u] ? mid[u] : 0];  // an open search: B has an entry
+      }
+#pragma unroll
+      for (int u = 0; u < kTsItems; ++u) {
+        if (lo[u] >= hi[u]) continue;
+        if ((uint64_t)c[u] < bound[u]) lo[u] = mid[u] + 1;
+        else hi[u] = mid[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kTsItems; ++u) {
+      const uint64_t i = i0 + u * kTsBlock + threadIdx.x;
+      if (i < total) ts[i] = lo[u];
     }
   }
 }
@@ -2352,12 +2386,10 @@ int tile_plan(uint64_t b_rows, uint64_t b_cols, uint32_t log2_cols, uint32_t bs,
 int launch_tile_starts(const DevCsr &B, uint32_t logW, uint32_t T1, uint32_t *ts,
                        hipStream_t s, const uint32_t *base) {
   if (B.rows == 0) return OC_OK;
-  uint32_t logP = 0;
-  while (logP < 6 && (1u << logP) < T1) ++logP;
-  const uint32_t rows_per_wg = 4u * (64u >> logP);
+  const uint64_t total = (uint64_t)B.rows * T1;
   hipLaunchKernelGGL(k_tile_starts,
-                     dim3(std::min<uint32_t>(cdiv(B.rows, rows_per_wg), 1u << 20)), dim3(256),
-                     0, s, B.rp, B.ci, (uint32_t)B.rows, logW, T1, base, ts, logP);
+                     dim3((uint32_t)std::min<uint64_t>((total + kTsTile - 1) / kTsTile, 1u << 16)),
+                     dim3(kTsBlock), 0, s, B.rp, B.ci, total, logW, T1, base, ts);
   LAUNCH_CHECK();
   return OC_OK;
 }
