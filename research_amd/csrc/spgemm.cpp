@@ -13,11 +13,11 @@
 #include <cstring>
 #include <initializer_list>
 #include <map>
-#include <mutex>
 #include <sstream>
 #include <string>
 #include <vector>
 
+#include "host_page.hpp"
 #include "launch.hpp"
 
 using namespace oc;
@@ -180,52 +180,6 @@ struct Marks {
         total += ms;
       }
     }
-  }
-};
-
-// A pinned host page that kernels write small results to (k_publish): word
-// 0 is the flag, the data start at word 16.
-// A handle takes its page on its first run and gives it back when it is
-// destroyed, with no work in flight; up to kIdle pages wait for the next
-// handles (allocating and freeing one costs about 100 us).
-struct HostPage {
-  static constexpr uint32_t kWords = 24 * 1024, kData = 16, kIdle = 16;
-  uint32_t *p = nullptr, seq = 0;
-  struct Idle {
-    std::mutex mu;
-    std::vector<uint32_t *> pages;
-  };
-  static Idle &idle() {
-    static Idle *i = new Idle();  // never destroyed: freed at process exit
-    return *i;
-  }
-  hipError_t take() {
-    if (p) return hipSuccess;
-    {
-      Idle &i = idle();
-      std::lock_guard<std::mutex> lk(i.mu);
-      if (!i.pages.empty()) {
-        p = i.pages.back();
-        i.pages.pop_back();
-      }
-    }
-    if (!p) {
-      const hipError_t e = hipHostMalloc((void **)&p, kWords * 4, hipHostMallocPortable);
-      if (e != hipSuccess) {
-        p = nullptr;
-        return e;
-      }
-    }
-    p[0] = seq = 0;
-    return hipSuccess;
-  }
-  void give() {
-    if (!p) return;
-    Idle &i = idle();
-    std::lock_guard<std::mutex> lk(i.mu);
-    if (i.pages.size() < kIdle) i.pages.push_back(p);
-    else (void)hipHostFree(p);
-    p = nullptr;
   }
 };
 
