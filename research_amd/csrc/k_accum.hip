@@ -956,6 +956,17 @@ __device__ __forceinline__ void for_bucket(const uint32_t *ck, uint32_t s0, uint
 // taken: their rows come from skewed structures that crowd the buckets and
 // need U = 12, 121 registers a lane; R-MAT 2^18's took 2324 us so, 1288 by
 // the table.
+// Neither are rows with more than kCrowded products in one bucket: each of
+// them is compared with all the others, one after another, and a lane waits
+// for every read.  The columns of a neighbourhood share a bucket once a single
+// far link widens the row's span, so such rows are common.  262,144 rows with
+// a band of 9, 11 or 13 entries and one far link (up to 81, 121 or 169
+// products in a bucket) took 1566, 2931 and 4884 us with a limit of 192
+// products, 438, 503 and 568 by the table after the count (637, 644 and 660
+// when all rows went by a table with a radix sort).  At the limit both cost
+// about the same (256 products in 8 or 4 columns, 16 and 25 in a bucket: 631
+// and 588 us with 24, 639 and 749 with 32, 719 and 591 with 16); uniform rows
+// have at most about 8 in a bucket.
 //
 // LDS: header, bucket starts and duplicate counts (u16, 4 BS each), then the
 // products' columns and values in bucket order.
@@ -963,7 +974,7 @@ template <int BS>
 struct SortRows {
   static constexpr int U = 5;                      // products per lane at most
   static constexpr int kLogBuckets = __builtin_ctz(BS) + 2;
-  static constexpr uint32_t kCrowded = 192;        // most products of one bucket
+  static constexpr uint32_t kCrowded = 24;         // most products of one bucket
   static constexpr uint32_t off_start = 1280, off_dup = off_start + 8 * BS + 8,
                             off_val = off_dup + 8 * BS + 8;
   __host__ __device__ static uint32_t capacity(uint32_t bytes) {

@@ -1,0 +1,58 @@
+"""A stage's time on either side of a rule that picks a route: products that
+differ little may not differ much in time.  Stage times are the library's own
+(HIP events), the least of several runs of both, taken in turn."""
+import numpy as np
+import pytest
+
+from helpers import log
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(gpu, rows, cols, ro, ci, seed=0):
+    rng = np.random.default_rng(seed)
+    return gpu.CSR(rows, cols, np.asarray(ro, np.uint32), np.asarray(ci, np.uint32),
+                   rng.uniform(-1, 1, len(ci)).astype(np.float32)).upload()
+
+
+def _spread(gpu, rows, cols, k):
+    """k entries a row, one in each of k equal column ranges."""
+    w = cols // k
+    ci = np.arange(k) * w + np.random.default_rng(k).integers(0, w, (rows, k))
+    return _csr(gpu, rows, cols, np.arange(rows + 1) * k, ci.ravel())
+
+
+def _band_and_link(gpu, n, half):
+    """A band of 2 half + 1 entries and one entry anywhere, a row."""
+    rng = np.random.default_rng(half)
+    base = np.clip(np.arange(n), half, n - 1 - half)[:, None] + np.arange(-half, half + 1)
+    m = np.sort(np.concatenate([base, rng.integers(0, n, (n, 1))], 1), 1)
+    keep = np.ones(m.shape, bool)
+    keep[:, 1:] = m[:, 1:] != m[:, :-1]
+    return _csr(gpu, n, n, np.r_[0, np.cumsum(keep.sum(1))], m[keep])
+
+
+def _stage_ms(gpu, stage, workflow, pairs):
+    sps = []
+    for _ in pairs:
+        sp = gpu.SpGEMM(gpu.Config(use_ultrasparse_workflow=0))
+        sp.set_workflow(workflow)
+        sps.append(sp)
+    ms = [np.inf] * len(pairs)
+    for i in range(9):
+        for k, (sp, (A, B)) in enumerate(zip(sps, pairs)):
+            sp.run(A, B)
+            if i >= 2:
+                ms[k] = min(ms[k], sp.timer_ms(stage))
+    log(f"{stage}: {', '.join(f'{m:.3f}' for m in ms)} ms")
+    return ms
+
+
+def test_clustered_hash_rows(gpu):
+    """Rows with most of their products in one neighbourhood and one far
+    link: 196 products a row may not take twice as long as 324 (they took
+    ten times as long while crowded buckets were sorted by comparison)."""
+    log("case: clustered hash rows")
+    M = [_band_and_link(gpu, 1 << 17, half) for half in (6, 8)]
+    few, more = _stage_ms(gpu, "numeric_hash", 0, [(m, m) for m in M])
+    assert few < 2 * more
