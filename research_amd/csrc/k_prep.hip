@@ -965,8 +965,16 @@ int launch_hll_merge(int log_p, const DevCsr &A, const uint8_t *hll,
   uint32_t *heavy_list = heavy_count + 16;
   OC_TRY(launch_fill_u32(heavy_count, 1, 0u, s));
   const uint32_t rows = (uint32_t)A.rows;
-  const uint32_t heavy = 512;  // entries one wave merges
   const uint32_t ntasks = mode == 0 ? rows : nsamples;
+  // Entries one wave merges; a longer row is listed, by an atomic, and taken
+  // by a workgroup, one for each CU.  The list is quick for a few rows: with
+  // 512 instead of 2048, the 648 samples of R-MAT 2^13 save 30 us, as no wave
+  // is left alone with a long row.  It is slow for many: 100,000 rows of 600
+  // entries took 2296 us by the list and 406 by the waves.  At most one row in
+  // 512 / mean is longer than 512 entries, so 512 holds where that bound is
+  // no more than eight rows a workgroup.
+  const double may_list = (double)A.nnz / (double)A.rows * (double)ntasks / 512.0;
+  const uint32_t heavy = may_list <= 8.0 * tables().num_cu ? 512u : 2048u;
   dim3 grid(std::max<uint32_t>(1, std::min<uint32_t>(cdiv(ntasks, 4), 1u << 18)));
   dim3 hgrid(std::max<uint32_t>(1, tables().num_cu));
 #define GO(L, M)                                                               \

@@ -56,3 +56,14 @@ def test_clustered_hash_rows(gpu):
     M = [_band_and_link(gpu, 1 << 17, half) for half in (6, 8)]
     few, more = _stage_ms(gpu, "numeric_hash", 0, [(m, m) for m in M])
     assert few < 2 * more
+
+
+def test_sketch_merge_of_many_long_rows(gpu):
+    """40,000 rows of 520 entries against 500: a few percent more sketches (it
+    was several times the time while every row above 512 went to the list of
+    rows that a workgroup takes)."""
+    log("case: sketch merge of many long rows")
+    B = _spread(gpu, 100_000, 100_000, 1)
+    shorter, longer = _stage_ms(gpu, "est_hll_merge", 1,
+                                [(_spread(gpu, 40_000, 100_000, k), B) for k in (500, 520)])
+    assert longer < 2 * shorter

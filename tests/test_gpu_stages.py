@@ -46,6 +46,8 @@ MATS = {
     "hubs": _hubs,
     "rmat13": lambda ra: ra.CSR.rmat(13, 16 << 13, seed=1),
     "er": lambda ra: ra.CSR.erdos_renyi(5000, 30.0, seed=2),
+    # so many rows of 513 to 2048 entries that waves merge their sketches
+    "long": lambda ra: ra.CSR.erdos_renyi(2000, 800.0, seed=4),
     "rect": lambda ra: ra.CSR.rect_band(3000, 50000, 8.0, 0.3, 4096, 8, vtype=1, seed=3),
 }
 
@@ -100,11 +102,12 @@ def test_murmur3_cols(gpu):
 
 
 @pytest.mark.parametrize("log_p", [5, 6])
-@pytest.mark.parametrize("name", ["rmat13", "er", "rect", "hubs"])
+@pytest.mark.parametrize("name", ["rmat13", "er", "rect", "hubs", "long"])
 def test_hll_build_estimate_sample(gpu, name, log_p):
     """Sketches, per-row estimates and samples bit-exact.  `hubs` has rows
-    of 2049, 6000 and 40000 entries: rows above 2048 entries are merged by
-    a whole workgroup each (the heavy-row kernel), in both modes."""
+    of 513 to 40000 entries: the longest are merged by a whole workgroup each
+    (the heavy-row kernel) in both modes, those above 2048 entries always
+    and those above 512 where few rows can be that long."""
     log(f"case: hll {name} log_p={log_p}")
     A, B = _pair(gpu, name)
     if name == "hubs":
