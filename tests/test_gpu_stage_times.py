@@ -67,3 +67,29 @@ def test_sketch_merge_of_many_long_rows(gpu):
     shorter, longer = _stage_ms(gpu, "est_hll_merge", 1,
                                 [(_spread(gpu, 40_000, 100_000, k), B) for k in (500, 520)])
     assert longer < 2 * shorter
+
+
+def _two_lengths(gpu, rows, cols, long, rate):
+    """A share of the rows with `long` entries, the others with two."""
+    rng = np.random.default_rng(1)
+    n = np.where(rng.random(rows) < rate, long, 2)
+    ro = np.r_[0, np.cumsum(n)]
+    ci = np.empty(ro[-1], np.int64)
+    for k in (2, long):
+        r = np.flatnonzero(n == k)
+        w = cols // k
+        ci[(ro[r][:, None] + np.arange(k)).ravel()] = \
+            (np.arange(k) * w + rng.integers(0, w, (len(r), k))).ravel()
+    return _csr(gpu, rows, cols, ro, ci)
+
+
+def test_analysis_of_many_long_rows(gpu):
+    """Half a million rows, one in twenty of 520 entries against 500: a few
+    percent more entries (it was twice the time while rows of 512 entries
+    were listed for a workgroup each at a mean of 28)."""
+    log("case: analysis of many long rows")
+    B = _spread(gpu, 1 << 18, 1 << 18, 1)
+    shorter, longer = _stage_ms(gpu, "analysis_product_calc", 1,
+                                [(_two_lengths(gpu, 1 << 19, 1 << 18, k, 0.05), B)
+                                 for k in (500, 520)])
+    assert longer < 1.5 * shorter
