@@ -512,28 +512,28 @@ __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uin
   const uint32_t wid =
       NW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t step = NW / share * kWave, sub = wid % share;
-  uint32_t c0 = a0 + wid / share * kWave;
-  if (c0 >= a1) return;
+  EntryWalk c(a0, a1, wid / share * kWave);  // the chunk's first entry
+  if (!c.has(0)) return;
   auto add = [](uint32_t x, uint32_t y) { return x + y; };
   // this chunk's B row bounds and A values, the next chunk's columns
   uint32_t bs = 0, be = 0, kn = 0;
   T av = T(0);
-  if (c0 + lane < a1) {
-    const uint32_t k = a.a_ci[c0 + lane];
-    if (VALS) av = a.a_v[c0 + lane];
+  if (c.has(lane)) {
+    const uint32_t k = a.a_ci[c.at + lane];
+    if (VALS) av = a.a_v[c.at + lane];
     bs = a.b_rp[k];
     be = a.b_rp[k + 1];
   }
-  if (c0 + step + lane < a1) kn = a.a_ci[c0 + step + lane];
+  if (c.has(step + lane)) kn = a.a_ci[c.at + step + lane];
   for (;;) {
-    const uint32_t cn = c0 + step;
+    c.skip(step);
     uint32_t bsn = 0, ben = 0;
     T avn = T(0);
-    if (cn + lane < a1) {
+    if (c.has(lane)) {
       bsn = a.b_rp[kn];
       ben = a.b_rp[kn + 1];
-      if (VALS) avn = a.a_v[cn + lane];
-      if (cn + step + lane < a1) kn = a.a_ci[cn + step + lane];
+      if (VALS) avn = a.a_v[c.at + lane];
+      if (c.has(step + lane)) kn = a.a_ci[c.at + step + lane];
     }
     const uint32_t len = be - bs > skip ? 0u : be - bs;
     const uint32_t incl = wave_incl_scan(len, 0u, add);
@@ -553,24 +553,23 @@ __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uin
         if (b + u < b1)  // uniform
           ok[u] = flat_owner<VALS>((b + u) * kWave, P, len, ex, base, av, q[u], pa[u]);
       }
-      uint32_t c[U];
+      uint32_t col[U];
       T v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        c[u] = 0;
+        col[u] = 0;
         v[u] = T(0);
         if (ok[u]) {
-          c[u] = a.b_ci[q[u]];
+          col[u] = a.b_ci[q[u]];
           if (VALS) v[u] = a.b_v[q[u]];
         }
       }
       double pv[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) pv[u] = VALS ? product_pz((double)pa[u], (double)v[u]) : 0.0;
-      if (!f(c, pv, ok)) return;
+      if (!f(col, pv, ok)) return;
     }
-    if (cn >= a1) return;
-    c0 = cn;
+    if (!c.has(0)) return;
     bs = bsn;
     be = ben;
     av = avn;
@@ -608,11 +607,11 @@ template <int BS, typename KA>
 __device__ __forceinline__ uint32_t list_longer(const KA &a, uint32_t a0, uint32_t a1,
                                                 uint32_t longest, uint32_t *count,
                                                 uint32_t *list, uint32_t cap) {
-  for (uint32_t j = a0 + threadIdx.x; j < a1; j += BS) {
-    const uint32_t k = a.a_ci[j];
+  for (EntryWalk j(a0, a1, threadIdx.x); j.has(0); j.skip(BS)) {
+    const uint32_t k = a.a_ci[j.at];
     if (a.b_rp[k + 1] - a.b_rp[k] > longest) {
       const uint32_t idx = atomicAdd(count, 1u);
-      if (idx < cap) list[idx] = j;
+      if (idx < cap) list[idx] = j.at;
     }
   }
   __syncthreads();

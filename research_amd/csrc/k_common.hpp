@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #include "dev_common.hpp"
+#include "entry_walk.hpp"
 #include "launch.hpp"
 
 namespace oc {

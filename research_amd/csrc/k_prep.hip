@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "dev_common.hpp"
+#include "entry_walk.hpp"
 #include "launch.hpp"
 
 namespace oc {
@@ -209,10 +210,10 @@ __global__ __launch_bounds__(kAnaBlock) void k_analysis(
       }
     } else {
       AnaAcc acc;
-      uint32_t j = s + lig;
-      for (; j + 3 * G < e; j += 4 * G) {  // four independent gathers in flight
-        const uint32_t k0 = a_ci[j], k1 = a_ci[j + G], k2 = a_ci[j + 2 * G],
-                       k3 = a_ci[j + 3 * G];
+      EntryWalk w(s, e, lig);
+      for (; w.has(3 * G); w.skip(4 * G)) {  // four independent gathers in flight
+        const uint32_t k0 = a_ci[w.at], k1 = a_ci[w.at + G], k2 = a_ci[w.at + 2 * G],
+                       k3 = a_ci[w.at + 3 * G];
         const uint4 v0 = info[k0], v1 = info[k1], v2 = info[k2], v3 = info[k3];
         acc.add(v0);
         acc.add(v1);
@@ -221,9 +222,9 @@ __global__ __launch_bounds__(kAnaBlock) void k_analysis(
       }
       // the rest (at most three), together: index 0 stands in for none
       {
-        const bool h0 = j < e, h1 = j + G < e, h2 = j + 2 * G < e;
-        const uint32_t k0 = h0 ? a_ci[j] : 0u, k1 = h1 ? a_ci[j + G] : 0u,
-                       k2 = h2 ? a_ci[j + 2 * G] : 0u;
+        const bool h0 = w.has(0), h1 = w.has(G), h2 = w.has(2 * G);
+        const uint32_t k0 = h0 ? a_ci[w.at] : 0u, k1 = h1 ? a_ci[w.at + G] : 0u,
+                       k2 = h2 ? a_ci[w.at + 2 * G] : 0u;
         const uint4 none = make_uint4(0u, 0xFFFFFFFFu, 0u, 0u);
         const uint4 v0 = h0 ? info[k0] : none, v1 = h1 ? info[k1] : none,
                     v2 = h2 ? info[k2] : none;
@@ -283,17 +284,17 @@ __global__ __launch_bounds__(kLongBlock) void k_analysis_long(
     const uint32_t r = long_rows[i];
     const uint32_t s = a_rp[r], e = a_rp[r + 1];
     AnaAcc acc;
-    uint32_t j = s + threadIdx.x;
-    for (; j + 3 * kLongBlock < e; j += 4 * kLongBlock) {
-      const uint32_t k0 = a_ci[j], k1 = a_ci[j + kLongBlock], k2 = a_ci[j + 2 * kLongBlock],
-                     k3 = a_ci[j + 3 * kLongBlock];
+    EntryWalk w(s, e, threadIdx.x);
+    for (; w.has(3 * kLongBlock); w.skip(4 * kLongBlock)) {
+      const uint32_t k0 = a_ci[w.at], k1 = a_ci[w.at + kLongBlock],
+                     k2 = a_ci[w.at + 2 * kLongBlock], k3 = a_ci[w.at + 3 * kLongBlock];
       const uint4 v0 = info[k0], v1 = info[k1], v2 = info[k2], v3 = info[k3];
       acc.add(v0);
       acc.add(v1);
       acc.add(v2);
       acc.add(v3);
     }
-    for (; j < e; j += kLongBlock) acc.add(info[a_ci[j]]);
+    for (; w.has(0); w.skip(kLongBlock)) acc.add(info[a_ci[w.at]]);
     const uint32_t prod = group_sum(acc.prod, kWave);
     const uint32_t mb = group_max(acc.mb, kWave);
     const uint32_t lo = group_min(acc.lo, kWave);
@@ -684,18 +685,19 @@ int launch_murmur(const uint32_t *cols, uint32_t *out, uint64_t n, hipStream_t s
 // longest row 39,618 entries: 670 -> 196 us; 2^18: 260 -> 58 us).
 constexpr uint32_t kHllLong = 512;
 
-// f(column) over entries j, j + step, ... < e, four loads in flight
+// f(column) over the walk's entries, step apart, four loads in flight
 template <typename F>
-__device__ __forceinline__ void hll_entries(const uint32_t *__restrict__ ci, uint32_t j,
-                                            uint32_t e, uint32_t step, F &&f) {
-  for (; j < e && e - j > 3 * step; j += 4 * step) {
-    const uint32_t c0 = ci[j], c1 = ci[j + step], c2 = ci[j + 2 * step], c3 = ci[j + 3 * step];
+__device__ __forceinline__ void hll_entries(const uint32_t *__restrict__ ci, EntryWalk w,
+                                            uint32_t step, F &&f) {
+  for (; w.has(3 * step); w.skip(4 * step)) {
+    const uint32_t c0 = ci[w.at], c1 = ci[w.at + step], c2 = ci[w.at + 2 * step],
+                   c3 = ci[w.at + 3 * step];
     f(c0);
     f(c1);
     f(c2);
     f(c3);
   }
-  for (; j < e; j += step) f(ci[j]);
+  for (; w.has(0); w.skip(step)) f(ci[w.at]);
 }
 
 template <int LOGP>
@@ -733,7 +735,7 @@ __global__ __launch_bounds__(256) void k_hll_build(const uint32_t *__restrict__ 
       } else {
         for (int i = lig; i < P; i += 16) regs[g][i] = 0;
         wave_sync();
-        hll_entries(ci, s + lig, e, 16, [&](uint32_t c) { into(regs[g], c); });
+        hll_entries(ci, EntryWalk(s, e, lig), 16, [&](uint32_t c) { into(regs[g], c); });
         wave_sync();
         store(regs[g], (uint32_t)r, lig);
       }
@@ -744,7 +746,7 @@ __global__ __launch_bounds__(256) void k_hll_build(const uint32_t *__restrict__ 
       for (int i = threadIdx.x; i < P; i += 256) regs[k][i] = 0;
       __syncthreads();
       const uint32_t lr = long_rows[k];
-      hll_entries(ci, rp[lr] + threadIdx.x, rp[lr + 1], 256,
+      hll_entries(ci, EntryWalk(rp[lr], rp[lr + 1], threadIdx.x), 256,
                   [&](uint32_t c) { into(regs[k], c); });
     }
     __syncthreads();
@@ -827,13 +829,13 @@ __device__ __forceinline__ uint32_t hll_merge_range(const uint32_t *a_ci,
   // reads nothing and is the neutral 0
   constexpr int U = 8;
   uint32_t m = 0;
-  for (uint32_t j = s + sk; j < e; j += U * S) {
+  for (EntryWalk j(s, e, sk); j.has(0); j.skip(U * S)) {
     uint32_t k[U], v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) k[u] = e - j > (uint32_t)(u * S) ? a_ci[j + u * S] : 0u;
+    for (int u = 0; u < U; ++u) k[u] = j.has(u * S) ? a_ci[j.at + u * S] : 0u;
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      v[u] = e - j > (uint32_t)(u * S)
+      v[u] = j.has(u * S)
                  ? reinterpret_cast<const uint32_t *>(hll + (uint64_t)k[u] * P)[w]
                  : 0u;
 #pragma unroll
@@ -907,9 +909,9 @@ __global__ __launch_bounds__(1024) void k_hll_merge_heavy(
       r = (uint32_t)(x % rows);
     }
     const uint32_t s = a_rp[r], e = a_rp[r + 1];
-    const uint32_t per = (e - s + 15) / 16;
-    const uint32_t ws = s + wid * per, we = min(e, ws + per);
-    uint32_t m = hll_merge_range<LOGP>(a_ci, hll, ws < e ? ws : e, ws < e ? we : e, lane);
+    const uint32_t per = (e - s) / 16 + ((e - s) % 16 != 0);
+    const EntryWalk mine(s, e, wid * per);  // this wave's sixteenth
+    uint32_t m = hll_merge_range<LOGP>(a_ci, hll, mine.at, mine.at + min(mine.left, per), lane);
     if (lane < W) part[wid][lane] = m;
     __syncthreads();
     if (wid == 0) {
