@@ -5,7 +5,7 @@
 
 #include <cstdint>
 #include <mutex>
-#include <vector>
+#include <type_traits>
 
 namespace oc {
 
@@ -23,23 +23,22 @@ struct HostPage {
   static constexpr unsigned kFlags =
       hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
   uint32_t *p = nullptr, seq = 0;
+  // Never destroyed, and without the heap: give() runs in destructors.
   struct Idle {
     std::mutex mu;
-    std::vector<uint32_t *> pages;
+    uint32_t *pages[kIdle], n = 0;
   };
   static Idle &idle() {
-    static Idle *i = new Idle();  // never destroyed: freed at process exit
-    return *i;
+    static_assert(std::is_trivially_destructible<Idle>::value, "outlives every handle");
+    static Idle i;
+    return i;
   }
   hipError_t take() {
     if (p) return hipSuccess;
     {
       Idle &i = idle();
       std::lock_guard<std::mutex> lk(i.mu);
-      if (!i.pages.empty()) {
-        p = i.pages.back();
-        i.pages.pop_back();
-      }
+      if (i.n) p = i.pages[--i.n];
     }
     if (!p) {
       const hipError_t e = hipHostMalloc((void **)&p, kWords * 4, kFlags);
@@ -53,10 +52,15 @@ struct HostPage {
   }
   void give() {
     if (!p) return;
-    Idle &i = idle();
-    std::lock_guard<std::mutex> lk(i.mu);
-    if (i.pages.size() < kIdle) i.pages.push_back(p);
-    else (void)hipHostFree(p);
+    {
+      Idle &i = idle();
+      std::lock_guard<std::mutex> lk(i.mu);
+      if (i.n < kIdle) {
+        i.pages[i.n++] = p;
+        p = nullptr;
+      }
+    }
+    if (p) (void)hipHostFree(p);
     p = nullptr;
   }
 };

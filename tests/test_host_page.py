@@ -17,8 +17,17 @@ ROCM = "/opt/rocm"
 PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 #include <vector>
 #include "host_page.hpp"
+
+static unsigned news = 0;  // heap allocations by C++ code
+void *operator new(std::size_t n) {
+  ++news;
+  return std::malloc(n);
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
 
 static std::vector<unsigned> flags;
 static unsigned mallocs = 0, frees = 0;
@@ -37,8 +46,11 @@ extern "C" hipError_t hipHostFree(void *p) {
 
 int main() {
   const unsigned kept = oc::HostPage::kIdle, n = kept + 3;
+  unsigned allocations = 0;
+  flags.reserve(3 * n);
   for (int round = 0; round < 2; ++round) {
     std::vector<oc::HostPage> pages(n);
+    const unsigned before = news;
     for (auto &p : pages) {
       if (p.take() != hipSuccess || !p.p || p.p[0] != 0 || p.seq != 0) return 1;
       uint32_t *first = p.p;
@@ -46,17 +58,18 @@ int main() {
       p.p[0] = p.seq = 7;
     }
     for (auto &p : pages) p.give();
+    allocations += news - before;
   }
   for (unsigned f : flags) std::printf("%x ", f);
-  std::printf("\n%u %u %u\n", mallocs, frees, kept);
+  std::printf("\n%u %u %u %u\n", mallocs, frees, kept, allocations);
   return 0;
 }
 """
 
 
-def build(tmp_path, extra=""):
+def build(tmp_path):
     src, exe = tmp_path / "page.cpp", tmp_path / "page"
-    src.write_text(extra + PROGRAM)
+    src.write_text(PROGRAM)
     subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include", f"-I{CSRC}",
                     "-o", str(exe), str(src), "-pthread"], check=True)
     return str(exe)
@@ -71,5 +84,8 @@ def test_page_is_coherent_and_pool_bounded(tmp_path):
         assert f & coherent and not f & non_coherent, hex(f)
         assert f & mapped and f & portable, hex(f)
     # 19 pages, 3 of them freed; then 16 from the pool and 3 new ones
-    mallocs, frees, kept = (int(x) for x in counts.split())
+    mallocs, frees, kept, allocations = (int(x) for x in counts.split())
     assert (mallocs, frees, kept) == (22, 6, 16)
+    # pages come and go without the heap: give() runs in a handle's destructor,
+    # where an allocation that fails would end the process
+    assert allocations == 0
