@@ -955,17 +955,21 @@ __device__ __forceinline__ void for_bucket(const uint32_t *ck, uint32_t s0, uint
 // taken: their rows come from skewed structures that crowd the buckets and
 // need U = 12, 121 registers a lane; R-MAT 2^18's took 2324 us so, 1288 by
 // the table.
-// Neither are rows with more than kCrowded products in one bucket: each of
-// them is compared with all the others, one after another, and a lane waits
-// for every read.  The columns of a neighbourhood share a bucket once a single
-// far link widens the row's span, so such rows are common.  262,144 rows with
-// a band of 9, 11 or 13 entries and one far link (up to 81, 121 or 169
-// products in a bucket) took 1566, 2931 and 4884 us with a limit of 192
-// products, 438, 503 and 568 by the table after the count (637, 644 and 660
-// when all rows went by a table with a radix sort).  At the limit both cost
-// about the same (256 products in 8 or 4 columns, 16 and 25 in a bucket: 631
-// and 588 us with 24, 639 and 749 with 32, 719 and 591 with 16); uniform rows
-// have at most about 8 in a bucket.
+// Nor are rows whose products outnumber the expected outputs (`hint`: the
+// count, or its estimate) by more than an eighth: the table has fewer entries
+// than the sort has products, and columns that meet are columns that crowd the
+// buckets.  (262,144 rows of 128 products in 8 columns: sorted 640 us, by the
+// table 395.  R-MAT 2^12 and 2^13, 256 threads, few rows that wait for memory:
+// 23.5 -> 13.8 and 19.7 -> 15.7 us.)
+// And a row with more than kCrowded products in one bucket goes back to the
+// table: each of them is compared with all the others, one after another, and
+// a lane waits for every read.  The columns of a neighbourhood share a bucket
+// once a single far link widens the row's span: 262,144 rows with a band of 13
+// entries and one far link, up to 169 products in a bucket, took 4884 us with
+// a limit of 192 products and 568 with 24, which is about where both ways cost
+// the same (660 when all rows went by a table with a radix sort; 395 now that
+// their outputs are known to be few).  Uniform rows have at most about 8 in a
+// bucket.
 //
 // LDS: header, bucket starts and duplicate counts (u16, 4 BS each), then the
 // products' columns and values in bucket order.
@@ -983,15 +987,15 @@ struct SortRows {
 
 template <int BS, typename T, bool EST>
 __device__ __forceinline__ bool num_sort_row(const KArgs<T> &a, uint32_t r, const RowHead &rh,
-                                             uint64_t off, uint32_t cap, uint32_t lds_bytes,
-                                             const KOut<T> &o) {
+                                             uint64_t off, uint32_t cap, uint32_t hint,
+                                             uint32_t lds_bytes, const KOut<T> &o) {
   using SR = SortRows<BS>;
   constexpr uint32_t NW = BS / kWave;
   constexpr int U = SR::U;
   extern __shared__ __align__(16) uint8_t smem[];
   const uint32_t nA = rh.a1 - rh.a0, P = rh.prod;
   const uint32_t nb = (P + kWave - 1) / kWave, per = (nb + NW - 1) / NW;
-  if (BS > 512 || nA == 0 || nA > kWave || P == 0 || per > (uint32_t)U || P > SR::capacity(lds_bytes) ||
+  if (P > hint + hint / 8 || BS > 512 || nA == 0 || nA > kWave || P == 0 || per > (uint32_t)U || P > SR::capacity(lds_bytes) ||
       rh.right - rh.left >= 0x80000000u)
     return false;
   uint32_t *hdr = reinterpret_cast<uint32_t *>(smem);
@@ -1176,9 +1180,10 @@ __device__ __forceinline__ void num_hash_row(KArgs<T> a,
   uint16_t *cnt = reinterpret_cast<uint16_t *>(smem + L.off_cnt);
   const uint32_t S = L.S;
   const RowHead rh = row_head(a, r);
+  const uint32_t hint = o.nnz_hint[r];
   const uint64_t off = o.off[r];
   const uint32_t cap = EST ? o.cap[r] : 0u;
-  if (num_sort_row<BS, T, EST>(a, r, rh, off, cap, L.bytes, o)) return;
+  if (num_sort_row<BS, T, EST>(a, r, rh, off, cap, hint, L.bytes, o)) return;
   for (uint32_t i = threadIdx.x; i < S; i += BS) {
     keys[i] = kEmpty;
     vals[i] = 0.0;
@@ -2628,12 +2633,14 @@ int launch_num_hash(int bin, const AccArgs &a, const uint32_t *rows,
   }
   const int kb = key_bits_for(a.B.cols);
   const bool est = o.cap != nullptr;
+  NumOut oh = o;
+  if (!oh.nnz_hint) oh.nnz_hint = a.products;  // read without a test in the kernel
 #define GO3(BS, T, E)                                                          \
   do {                                                                         \
     OC_TRY(set_lds(k_num_hash<BS, T, E>, L.bytes));                            \
     const BinGrid bg = bin_grid(sel, rows, nrows, k_num_hash<BS, T, E>, BS, L.bytes); \
     hipLaunchKernelGGL((k_num_hash<BS, T, E>), dim3(bg.grid), dim3(BS), L.bytes, \
-                       s, kargs<T>(a), bg.rows, bg.bounds, sel.err, L, kout<T>(o), kb, \
+                       s, kargs<T>(a), bg.rows, bg.bounds, sel.err, L, kout<T>(oh), kb, \
                        bg.claim);                                             \
   } while (0)
 #define GO(BS)                                            \

@@ -1,7 +1,8 @@
 """Numeric hash rows sorted by column without a table (num_sort_row) at the
 edges of what it takes: 63 to 65 A entries, as many products as a lane keeps
-(5 for each thread) and as the LDS of each table size holds, duplicates, empty
-B rows at the ends and in between, and buckets one below, at and one above
+(5 for each thread) and as the LDS of each table size holds, an eighth more
+products than outputs, duplicates, empty B rows at the ends and in between, and
+buckets one below, at and one above
 the crowding limit.  The structure is bit-exact; each value is a sum of at
 most 3 products, within 1e-12 (f64) and 1e-5 (f32) of the oracle's,
 condition-normalised."""
@@ -73,8 +74,10 @@ def test_limits(gpu, entries, vtype):
     rng = np.random.default_rng(entries)
     rows = []
     for p in _edges():
-        for share in (1.0, 0.57, 0.5):  # outputs per product: another table size
-            outputs = max(1, int(p * share))
+        # outputs: another table size, and about an eighth less than products
+        eighth = -(-8 * p // 9)
+        for outputs in {p, eighth - 1, eighth, eighth + 1, int(0.57 * p), p // 2}:
+            outputs = min(p, max(1, outputs))
             lengths = _lengths(rng, entries, p)
             pool = rng.choice(COLS, max(outputs, int(lengths.max())), replace=False)
             rows.append(_deal(pool, lengths))

@@ -58,6 +58,20 @@ def test_clustered_hash_rows(gpu):
     assert few < 2 * more
 
 
+def test_hash_rows_whose_products_meet(gpu):
+    """128 products a row in 8 columns or in columns of their own: a sixteenth
+    of the outputs may not cost half as much again (sorting the products cost
+    twice as much where they meet)."""
+    log("case: hash rows whose products meet")
+    rows, cols = 1 << 17, 1 << 20
+    A = _spread(gpu, rows, rows, 64)
+    rng = np.random.default_rng(2)
+    two = np.sort(np.argsort(rng.random((rows, 8)), 1)[:, :2], 1) * ((cols - 1) // 7)
+    meet = _csr(gpu, rows, cols, np.arange(rows + 1) * 2, two.ravel())
+    few, many = _stage_ms(gpu, "numeric_hash", 0, [(A, meet), (A, _spread(gpu, rows, cols, 2))])
+    assert few < 1.5 * many
+
+
 def test_sketch_merge_of_many_long_rows(gpu):
     """40,000 rows of 520 entries against 500: a few percent more sketches (it
     was several times the time while every row above 512 went to the list of
