@@ -2639,6 +2639,7 @@ int launch_num_hash(int bin, const AccArgs &a, const uint32_t *rows,
   do {                                                                         \
     OC_TRY(set_lds(k_num_hash<BS, T, E>, L.bytes));                            \
     const BinGrid bg = bin_grid(sel, rows, nrows, k_num_hash<BS, T, E>, BS, L.bytes); \
+    if (bg.claim && sel.clear) OC_TRY(zero_u32(bg.claim, 1, s));               \
     hipLaunchKernelGGL((k_num_hash<BS, T, E>), dim3(bg.grid), dim3(BS), L.bytes, \
                        s, kargs<T>(a), bg.rows, bg.bounds, sel.err, L, kout<T>(oh), kb, \
                        bg.claim);                                             \
@@ -2676,6 +2677,7 @@ int launch_num_dense(int dense_bin, const AccArgs &a, const uint32_t *rows,
   do {                                                                          \
     OC_TRY(set_lds(k_num_dense<BS, T, E>, lds));                                \
     const BinGrid bg = bin_grid(sel, rows, nrows, k_num_dense<BS, T, E>, BS, lds); \
+    if (bg.claim && sel.clear) OC_TRY(zero_u32(bg.claim, 1, s));                \
     hipLaunchKernelGGL((k_num_dense<BS, T, E>), dim3(bg.grid), dim3(BS), lds, s, \
                        kargs<T>(a), bg.rows, bg.bounds, sel.err, kout<T>(o), bg.claim); \
   } while (0)

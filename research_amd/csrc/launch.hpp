@@ -177,7 +177,9 @@ struct NumOut {
 struct RowSel {
   const uint32_t *bounds = nullptr;
   const uint32_t *err = nullptr;
-  uint32_t *claim = nullptr;  // this launch's row-claim counter (hash/dense bins), zeroed before it
+  // this launch's row-claim counter (hash/dense bins); zeroed before it, or
+  // by it with `clear`
+  uint32_t *claim = nullptr;
   // the bin's first list entry when the host knows it (eager runs, which
   // pass the bin's row count): bins with many workgroups per CU then run
   // one workgroup per row from rows + first
@@ -186,6 +188,7 @@ struct RowSel {
   // with many workgroups per CU then run about that many workgroups, each
   // striding over the bin's present rows, and claim nothing.
   uint32_t planned = 0;
+  bool clear = false;
 };
 
 // Symbolic: rows of one bin.  Overflowing rows (estimated-compaction hash

@@ -785,6 +785,11 @@ struct Run {
   int numeric_bins(const uint32_t *brows, const uint32_t *hoff, const NumOut &o,
                    bool window_bin13, const uint32_t *boff = nullptr) {
     const AccArgs a = acc();
+    // a value-only replay clears the counters of the bins that claim (small
+    // products have none), a run has cleared them all with its others
+    auto sel = [&](int b) {
+      return RowSel{boff + b, nullptr, claim_ctr + kClaimNumeric + b, hoff[b], 0, replay};
+    };
     auto stage = [&](const char *name, bool work) {
       if (work) mk.mark(name);
       else mk.none(name);
@@ -797,8 +802,7 @@ struct Run {
         return OC_ERR_INVALID;
       }
       if (boff)
-        OC_TRY(launch_num_hash(b, a, brows, n, o, s,
-                               RowSel{boff + b, nullptr, claim_ctr + kClaimNumeric + b, hoff[b]}));
+        OC_TRY(launch_num_hash(b, a, brows, n, o, s, sel(b)));
       else
         OC_TRY(launch_num_hash(b, a, brows + hoff[b], n, o, s));
     }
@@ -808,8 +812,7 @@ struct Run {
       const uint32_t n = hoff[b + 1] - hoff[b];
       if (!n) continue;
       if (boff)
-        OC_TRY(launch_num_dense(b - 7, a, brows, n, o, s,
-                                RowSel{boff + b, nullptr, claim_ctr + kClaimNumeric + b, hoff[b]}));
+        OC_TRY(launch_num_dense(b - 7, a, brows, n, o, s, sel(b)));
       else
         OC_TRY(launch_num_dense(b - 7, a, brows + hoff[b], n, o, s));
     }
@@ -2038,7 +2041,6 @@ int replay_impl(oc_spgemm *h, hipStream_t s) {
   const uint32_t keep_max = h->max_a_nnz;
   h->max_a_nnz = p.max_a_nnz;
   r.claim_ctr = p.err + 32;  // the plan's claim counters (no allocation here)
-  OC_TRY(launch_fill_u32(r.claim_ctr, Run::kClaims, 0u, s));
   int rc = r.numeric_bins(p.brows, p.hoff, p.o, true, p.boff2);
   if (rc == OC_OK) rc = r.band_numeric(p.o);
   h->max_a_nnz = keep_max;
