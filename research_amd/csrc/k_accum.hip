@@ -587,6 +587,13 @@ __device__ __forceinline__ void for_products(const KArgs<T> &a, uint32_t a0, uin
 // rows, however long, are then shared evenly by all waves.  R-MAT 2^18, 1024
 // threads: 1431 -> 1291 us.)
 constexpr uint32_t kFlatAvg = 64;
+// Symbolic hash rows besides need kFlatSym products and B rows of different
+// lengths.  Groups of equal rows end together, and a key is one compare-and-
+// swap, so finding the owners costs more than it saves there; below about 13 x
+// 13 products it does for any rows.  (131,072 Erdos-Renyi rows of mean degree 4
+// / 8 / 12 / 16 / 24: 160 / 186 / 228 / 317 / 878 us by groups, 196 / 214 / 239 /
+// 296 / 683 by products; 131,072 rows of 64 B rows of 10 each 288 and 440.)
+constexpr uint32_t kFlatSym = 160;
 
 // Waves per chunk of for_products: enough blocks of 64 products for each (U
 // at a time), and no more chunks at once than the row has.
@@ -676,7 +683,7 @@ __device__ __forceinline__ void sym_hash_row(KArgs<float> a,
   const int G = pick_group_lat<8>(a1 - a0, rh.prod, rh.maxb, BS);
   const int ngroups = BS / G, gid = threadIdx.x / G, lig = threadIdx.x % G;
   const uint32_t avg = a1 > a0 ? rh.prod / (a1 - a0) : 0u;
-  const bool flat = avg < kFlatAvg;
+  const bool flat = avg < kFlatAvg && rh.prod >= kFlatSym && rh.maxb > avg + avg / 8;
   if (use_bm) {
     auto mark = [&](uint32_t col) {
       const uint32_t c = col - blo;

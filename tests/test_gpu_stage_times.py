@@ -72,6 +72,26 @@ def test_hash_rows_whose_products_meet(gpu):
     assert few < 1.5 * many
 
 
+def test_symbolic_rows_of_equal_b_rows(gpu):
+    """64 B rows of 10 entries against 64 of 8 and 12 in turn, 640 products
+    each: equal rows are the easier case by at least a tenth (they took as long
+    while both were walked product by product)."""
+    log("case: symbolic hash rows, equal and unequal B rows")
+    rows, cols = 1 << 17, 1 << 20
+    A = _spread(gpu, rows, rows, 64)
+    n = np.where(np.arange(rows) % 2, 8, 12)
+    ro = np.r_[0, np.cumsum(n)]
+    ci = np.empty(ro[-1], np.int64)
+    for k in (8, 12):
+        r = np.flatnonzero(n == k)
+        w = cols // k
+        ci[(ro[r][:, None] + np.arange(k)).ravel()] = \
+            (np.arange(k) * w + np.random.default_rng(k).integers(0, w, (len(r), k))).ravel()
+    equal, unequal = _stage_ms(gpu, "symbolic_hash", 0,
+                               [(A, _spread(gpu, rows, cols, 10)), (A, _csr(gpu, rows, cols, ro, ci))])
+    assert equal < 0.9 * unequal
+
+
 def test_sketch_merge_of_many_long_rows(gpu):
     """40,000 rows of 520 entries against 500: a few percent more sketches (it
     was several times the time while every row above 512 went to the list of
