@@ -806,13 +806,18 @@ __device__ __forceinline__ void sym_hash_row(KArgs<float> a,
   }
 }
 
-template <int BS>
+// OWN: one workgroup per row (no bounds), a kernel of its own: inside the loops
+// of bin_rows the same rows took longer (131,072 dense rows of 2400 products
+// 421 us, as a kernel of its own 359; hash rows of 64 products 357 and 343).
+template <int BS, bool OWN = false>
 __global__ __launch_bounds__(BS) void k_sym_hash(KArgs<float> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, uint32_t S, uint32_t limit, uint32_t *__restrict__ nnz, uint32_t *ovf_rows, uint32_t *ovf_count,
     uint32_t *claim) {
-  bin_rows(bounds, claim, [&](uint32_t i) {
+  auto row = [&](uint32_t i) {
     sym_hash_row<BS>(a, rows[i], S, limit, nnz, ovf_rows, ovf_count);
-  });
+  };
+  if constexpr (OWN) row(blockIdx.x);
+  else bin_rows(bounds, claim, row);
 }
 
 // ========================================================= symbolic dense
@@ -889,13 +894,13 @@ __device__ __forceinline__ void sym_dense_row(KArgs<float> a,
   if (threadIdx.x == 0) nnz[r] = hdr[0];
 }
 
-template <int BS, bool WIN = false>
+template <int BS, bool WIN = false, bool OWN = false>
 __global__ __launch_bounds__(BS) void k_sym_dense(KArgs<float> a, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ bounds, uint32_t *__restrict__ nnz, const uint64_t *__restrict__ bmoff, uint4 *__restrict__ bm,
     uint32_t wbits, uint32_t *claim) {
-  bin_rows(bounds, claim, [&](uint32_t i) {
-    sym_dense_row<BS, WIN>(a, rows[i], nnz, bmoff, bm, wbits);
-  });
+  auto row = [&](uint32_t i) { sym_dense_row<BS, WIN>(a, rows[i], nnz, bmoff, bm, wbits); };
+  if constexpr (OWN) row(blockIdx.x);  // as in k_sym_hash
+  else bin_rows(bounds, claim, row);
 }
 
 // ========================================================== numeric hash
@@ -2571,9 +2576,10 @@ int launch_sym_hash(int bin, const AccArgs &a, const uint32_t *rows,
   do {                                                                        \
     OC_TRY(set_lds(k_sym_hash<BS>, lds));                                     \
     const BinGrid bg = bin_grid(sel, rows, nrows, k_sym_hash<BS>, BS, lds); \
-    hipLaunchKernelGGL(k_sym_hash<BS>, dim3(bg.grid), dim3(BS), lds, s, k,     \
-                       bg.rows, bg.bounds, S, std::min(limit, S), nnz,         \
-                       ovf_rows, ovf_count, bg.claim);                       \
+    OC_TRY(set_lds(k_sym_hash<BS, true>, lds));                                \
+    hipLaunchKernelGGL((bg.bounds ? k_sym_hash<BS> : k_sym_hash<BS, true>),    \
+                       dim3(bg.grid), dim3(BS), lds, s, k, bg.rows, bg.bounds, \
+                       S, std::min(limit, S), nnz, ovf_rows, ovf_count, bg.claim); \
   } while (0)
   BIN_DISPATCH(bin, GO)
 #undef GO
@@ -2593,9 +2599,10 @@ int launch_sym_dense(int dense_bin, const AccArgs &a, const uint32_t *rows,
   do {                                                                         \
     OC_TRY(set_lds(k_sym_dense<BS>, lds));                                     \
     const BinGrid bg = bin_grid(sel, rows, nrows, k_sym_dense<BS>, BS, lds); \
-    hipLaunchKernelGGL(k_sym_dense<BS>, dim3(bg.grid), dim3(BS), lds, s, k,     \
-                       bg.rows, bg.bounds, nnz, bmoff, (uint4 *)bm, 0u,         \
-                       bg.claim);                                             \
+    OC_TRY(set_lds(k_sym_dense<BS, false, true>, lds));                         \
+    hipLaunchKernelGGL((bg.bounds ? k_sym_dense<BS> : k_sym_dense<BS, false, true>), \
+                       dim3(bg.grid), dim3(BS), lds, s, k, bg.rows, bg.bounds,  \
+                       nnz, bmoff, (uint4 *)bm, 0u, bg.claim);                  \
   } while (0)
   BIN_DISPATCH(dense_bin, GO)
 #undef GO
