@@ -25,15 +25,20 @@ def _chk(gpu, rc):
 
 
 def _hubs(ra):
-    """Rows of every length class of the analysis: short rows, rows just
-    below and above the long-row cut of each lane-group width, and one hub
-    row of 40000 entries; a third of the rows (so of B's rows) are empty."""
+    """Rows of every length class of the analysis and the sketches: short
+    rows, rows just below and above the cuts at 256 (long rows of the
+    analysis at this mean length), 512 and 2048 entries, alone and several in
+    one block of 16 rows, and one hub row of 40000 entries; a third of the
+    rows (so of B's rows) are empty."""
     rng = np.random.default_rng(11)
     n = 50000
     lens = rng.integers(0, 24, n)
     lens[rng.random(n) < 0.33] = 0
-    for i, L in enumerate([127, 128, 129, 511, 512, 513, 1024, 1025, 2049, 6000, 40000]):
+    for i, L in enumerate([127, 128, 129, 255, 256, 257, 511, 512, 513, 1024, 1025, 2047, 2048,
+                           2049, 6000, 40000]):
         lens[100 + 97 * i] = L
+    lens[32016:32032] = [513, 0, 600, 3, 512, 700, 1500, 0, 0, 5, 520, 0, 900, 0, 514, 2100]
+    lens[40000:40016] = 530  # a block of 16 rows, each swept by the whole workgroup
     ro = np.zeros(n + 1, np.uint32)
     np.cumsum(lens, out=ro[1:])
     ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens]).astype(np.uint32)
