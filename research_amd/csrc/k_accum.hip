@@ -397,7 +397,8 @@ __device__ __forceinline__ uint32_t list_heavy(const KA &a, const RowHead &rh, u
 }
 
 // The rows of a bin kernel:
-//  - the workgroup's own (no bounds: one workgroup per row);
+//  - the workgroup's own (no bounds: one workgroup per row; the symbolic
+//    kernels have a form without this function for it);
 //  - without a claim counter, the rows [bounds[0], bounds[1]) by a stride of
 //    the grid (which is then about as many workgroups as rows);
 //  - else those rows in chunks claimed from *claim (zeroed before the
@@ -1468,7 +1469,7 @@ __global__ __launch_bounds__(BS) void k_num_hash(KArgs<T> a, const uint32_t *__r
 // lanes of a wave take consecutive entries of a B row, whose bits share a
 // word.  The waves then sweep 64 columns at a time, place the set ones by a
 // ballot and store them coalesced.  (131,072 banded rows of 33 x 33
-// products, f32: 498 -> 325 us.)
+// products, f32: 498 -> 325 us, and 221 with the products walked in blocks.)
 __device__ __forceinline__ double product_pz(double x, double y) {
 #pragma clang fp contract(off)  // one rounding more would keep the sign of an underflow
   const double p = x * y;

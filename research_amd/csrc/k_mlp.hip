@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kMlpBlock) void k_mlp_backward(
   {  // dW2[h1][h2]: wave w takes h1 tile w
     const int mt = w;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
+    for (int nt = 0; nt < 4; ++nt) {
       f4 acc = {0.f, 0.f, 0.f, 0.f};
       acc = mfma(ld_colk(s.H1, kS64, mt * 16, 0), ld_colk(sb.dZ2, kS64, nt * 16, 0), acc);
       acc = mfma(ld_colk(s.H1, kS64, mt * 16, 32), ld_colk(sb.dZ2, kS64, nt * 16, 32), acc);

@@ -59,7 +59,9 @@ static Tables derive_tables(const int32_t *conc_in, const int32_t *block_in) {
     // numeric hash: keys (4 B) + FP64 sums (8 B) + sort buffers (4 B per
     // slot) + 1280 B header/digit totals + 512 B of radix counters per wave
     t.hash_num[b] = b == 0 ? 0 : ((l - 1312 - nw * 512) / 16) & ~7u;
-    // dense numeric: FP64 sum + 1 bit per column
+    // dense numeric: an FP64 sum per column.  The limit also counts a bit per
+    // column and 768 bytes more than the sums take: it is the one of a layout
+    // with a bitmap, kept so that every row stays in its bin.
     t.dense_num[b] = b == 6 ? 0xFFFFFFFFu : (((l - 1024) * 8) / 65) & ~31u;
   }
   t.max_dense_sym_bin = 6;

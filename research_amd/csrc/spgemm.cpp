@@ -537,8 +537,7 @@ struct Run {
 
   // Counters of a run, cleared by one launch: [0..7] overflow counts, from
   // kCtlClaims on the row-claim counters of the persistent bin launches, one
-  // each
-  // (symbolic bin b: b, the recount of overflow rows: 14, numeric bin b:
+  // each (symbolic bin b: b, the recount of overflow rows: 14, numeric bin b:
   // 16 + b).  The overflow list follows at kCtlWords.
   static constexpr uint32_t kClaims = 30, kClaimRecount = 14, kClaimNumeric = 16;
   static constexpr uint32_t kCtlClaims = 16, kCtlWords = 64;
